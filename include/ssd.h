@@ -88,7 +88,8 @@ extern "C" {
  * F16S_LOCAL; the chain keeps them in f32 registers.  So the forward's last
  * bits depend on the launch plan, which depends on batch x heads and the
  * device's CU count: results are not bitwise invariant to batch slicing.
- * state_dtype SPLIT (at chunk 256) keeps every local state in f32. */
+ * state_dtype SPLIT (at chunk 256) keeps every local state in f32.  (None of
+ * this concerns the forwards that run as a chain walk, see ssd_forward.) */
 enum {
   SSD_DTYPE_F32 = 0,
   SSD_DTYPE_BF16 = 1,
@@ -256,7 +257,14 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
                    const void* prep, const ssd_epilogue* epilogue, void* stream);
 
 /* Whole SSD forward (K1, K0, K2, K3, K4 on one stream): the replacement for
- * SSDLayer._ssd_core (MR:123-162).  Launches, all on `stream`: at chunk 256
+ * SSDLayer._ssd_core (MR:123-162).  16-bit inputs at dstate 128 with an even
+ * number of heads per group, state_dtype SSD_DTYPE_F32 and enough (batch,
+ * head) chains times tokens run as a walk along the chains, 64 tokens a step
+ * with the state in f32 registers, so that no per-chunk state is stored
+ * (operands, then for few chains the end states of their segments, then the
+ * walk: two to four launches; the workspace is the same).  Its results differ
+ * from the stage kernels' by rounding; SSD_STATE_F16S (or SPLIT) as
+ * state_dtype keeps the stage kernels.  Otherwise, all on `stream`: at chunk 256
  * with 16-bit inputs K1 + K0 as one launch, then K2 + K3 as one state-chain
  * launch (the chain's mixed plan adds K3 over the chains it leaves as
  * segments) or K2 then K3 where the chains are too few, then K4: three or
@@ -271,9 +279,9 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * runs at 256 unless that workspace would be larger than the caller's
  * chunk's (see ssd_forward_chunk).  Every chunking evaluates the same linear
  * recurrence (MR:152-161), so this changes rounding only. */
-/* The chunk length ssd_forward (and ssd_forward_noalloc) runs d at for this
- * dtype and state_dtype: d->chunk, or 256 where the rule above applies; 0
- * for invalid dims.  Host-only.  No counterpart in the reference (its
+/* The chunk length ssd_forward (and ssd_forward_noalloc) runs d's stage
+ * kernels at, and sizes its workspace for, with this dtype and state_dtype:
+ * d->chunk, or 256 where the rule above applies; 0 for invalid dims.  Host-only.  No counterpart in the reference (its
  * block_len is the chunk); for callers that size the workspace at the chunk
  * actually run or time its kernels one by one. */
 int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype);
@@ -349,8 +357,9 @@ size_t ssd_layer_workspace_bytes(const ssd_dims* d, int dtype);
  * output slices x_in [b, L, h*P], z [b, L, h*P], bmat/cmat [b, L, g, N] and
  * dt_in [b, L, h] (all of dtype, any strides with unit innermost stride) to
  * out_proj's input y [b, L, h*P]:
- *   ssd_layer_prep, then the SSD core (K0, K2, K3, K4 of ssd_forward), with
- *   the skip D x and the gate silu(z) fused into K4's write of y.
+ *   ssd_layer_prep, then the SSD core (K0, K2, K3, K4 of ssd_forward, or its
+ *   chain walk), with the skip D x and the gate silu(z) fused into the one
+ *   write of y.
  * z_strides / y_strides are over [b, L, h*P].  d->chunk is MR's block_len
  * and only has to divide L: for 16-bit inputs with L % 256 == 0 and dstate
  * 64 / 128 the core runs at chunk 256, whose result equals every other

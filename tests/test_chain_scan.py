@@ -1,0 +1,244 @@
+"""The chain walk (csrc/ssd_chain_scan.hip): ssd_forward and ssd_layer on 16-bit
+inputs at d_state 128 with at least ten (chain, 64-token step) pairs per CU.
+
+GPU: against the float64 oracle (chunked evaluation at 64), at shapes that
+take one segment, segments whose entering state each workgroup forms itself
+(up to 4) and segments that state_passing finishes, with ragged last
+segments, both types, dt, an initial state, strided operands and state rows
+outside f16's range.  y within 2e-2 (the 16-bit tolerance); the final state,
+whose products run on hi + lo pairs of the input type, to f32 accuracy: the
+pair is within 2^-17 of each product, so 3e-5 of max|state| (as
+tests/test_gpu_parity.py holds chunk_state).
+
+CPU: the per-lane LDS address formulas, restated and pinned to the source."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ssd_oracle as O
+from test_address_bounds import inside, pin
+from workloadsuite_amd import ssd as S
+
+DEV = "cuda"
+F = "ssd_chain_scan.hip"
+
+
+def case(dtype, b, L, h, g, seed, scale=None):
+    gen = torch.Generator().manual_seed(seed)
+    X = torch.randn(b, L, h, 64, generator=gen)
+    if scale is not None:
+        X = X * scale
+    A = -torch.rand(b, L, h, generator=gen) * 0.2
+    B = torch.randn(b, L, g, 128, generator=gen) * 128 ** -0.5
+    C = torch.randn(b, L, g, 128, generator=gen) * 128 ** -0.5
+    dt = torch.rand(b, L, h, generator=gen) + 0.1
+    init = torch.randn(b, h, 64, 128, generator=gen)
+    return X.to(dtype), A, B.to(dtype), C.to(dtype), dt, init
+
+
+def check(Y, final, ref, fref, tol=2e-2):
+    torch.testing.assert_close(Y.double().cpu(), ref, rtol=tol, atol=tol)
+    torch.testing.assert_close(final.double().cpu(), fref, rtol=0, atol=3e-5 * fref.abs().max().item())
+
+
+SHAPES = [
+    # b, L, h, g: one segment (512 chains of 6 steps); 2-4 segments; more than
+    # four (16 chains of 193 steps); a prime number of steps; six heads per group
+    (8, 384, 64, 4),
+    (2, 2496, 64, 8),
+    (1, 12352, 16, 2),
+    (1, 64 * 67, 48, 1),
+    (3, 1088, 96, 16),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", SHAPES)
+@pytest.mark.parametrize("opts", [True, False])
+def test_forward(dtype, b, L, h, g, opts):
+    print("CASE chain walk", dtype, b, L, h, g, opts, flush=True)
+    X, A, B, C, dt, init = case(dtype, b, L, h, g, seed=L + h)
+    dt, init = (dt, init) if opts else (None, None)
+    hs = [0, 1, h // 2, h - 1]   # heads of the first, a middle and the last workgroup
+    grp = [k // (h // g) for k in hs]
+    ref, fref = O.ssd_chunked(X[:, :, hs], A[:, :, hs], B[:, :, grp], C[:, :, grp], 64,
+                              dt=None if dt is None else dt[:, :, hs], initial_states=None if init is None else init[:, hs])
+    d = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    Y, final = S.ssd_forward(d(X), d(A), d(B), d(C), 64, dt=d(dt), initial_states=d(init), return_final_states=True)
+    torch.cuda.synchronize()
+    assert torch.isfinite(Y).all() and torch.isfinite(final).all()
+    check(Y[:, :, hs], final[:, hs], ref, fref)
+
+
+@pytest.mark.gpu
+def test_state_rows_outside_f16():
+    """x scaled per column p over 16 decades (states from ~1e-9 to ~1e6): rows
+    take their power-of-two scale.  Each column of y against its own scale."""
+    print("CASE chain walk, wide rows", flush=True)
+    col = torch.logspace(-9, 6, 64)
+    X, A, B, C, dt, init = case(torch.bfloat16, 8, 384, 64, 4, seed=5, scale=col)
+    init = init * col[:, None]
+    hs = [0, 31, 63]
+    grp = [k // 16 for k in hs]
+    ref, fref = O.ssd_chunked(X[:, :, hs], A[:, :, hs], B[:, :, grp], C[:, :, grp], 64, dt=dt[:, :, hs],
+                              initial_states=init[:, hs])
+    Y, final = S.ssd_forward(*(t.to(DEV) for t in (X, A, B, C)), 64, dt=dt.to(DEV), initial_states=init.to(DEV),
+                             return_final_states=True)
+    torch.cuda.synchronize()
+    check(Y[:, :, hs].double().cpu() / col, final[:, hs].double().cpu() / col[:, None].double(), ref / col,
+          fref / col[:, None])
+
+
+@pytest.mark.gpu
+def test_strided_operands_match_contiguous_ones():
+    """x, B, C as column slices of a wider tensor, A and dt transposed: the bits of the contiguous call."""
+    print("CASE chain walk, strides", flush=True)
+    X, A, B, C, dt, init = (t.to(DEV) for t in case(torch.float16, 2, 1280, 64, 4, seed=9))
+    wide = torch.zeros(2, 1280, 64 * 64 + 2 * 4 * 128 + 16, device=DEV, dtype=torch.float16)
+    xs, bs, cs = wide[..., 8:8 + 4096], wide[..., 4104:4104 + 512], wide[..., 4616:4616 + 512]
+    xs.copy_(X.flatten(2)), bs.copy_(B.flatten(2)), cs.copy_(C.flatten(2))
+    At, dtt = A.transpose(1, 2).contiguous().transpose(1, 2), dt.transpose(1, 2).contiguous().transpose(1, 2)
+    Y0, f0 = S.ssd_forward(X, A, B, C, 64, dt=dt, initial_states=init, return_final_states=True)
+    Y1, f1 = S.ssd_forward(xs.unflatten(2, (64, 64)), At, bs.unflatten(2, (4, 128)), cs.unflatten(2, (4, 128)), 64, dt=dtt,
+                           initial_states=init, return_final_states=True)
+    torch.cuda.synchronize()
+    assert torch.equal(Y0, Y1) and torch.equal(f0, f1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)])
+def test_layer_span(dtype, b, L, h, g):
+    """The gated variant (four heads per workgroup, two, and with segments)
+    against the stage entry points on the same prepared operands, 2e-2."""
+    from test_layer_kernels import layer_case, split
+    print("CASE chain walk, layer span", dtype, b, L, h, g, flush=True)
+    proj, prm = layer_case(dtype, b=b, L=L, h=h, P=64, g=g, N=128)
+    x, z, B, C, dt = split(proj.to(DEV), h, 64, g, 128)
+    p = {k: v.to(DEV) for k, v in prm.items()}
+    y = S.ssd_layer(x, z, B, C, dt, p["conv_w"], p["conv_b"], p["dt_bias"], p["A_log"], p["D"], 64, h)
+    X, dto, Acs, dec = S.layer_prep(x, dt, p["conv_w"], p["conv_b"], p["dt_bias"], p["A_log"], 64, h)
+    S_in, _ = S.chunk_state_passing(X, B, Acs, dec, dt=dto)
+    ref = S.chunk_scan(X, B, C, Acs, S_in, dt=dto, D=p["D"], z=z.reshape(b, L, h, 64))
+    torch.cuda.synchronize()
+    torch.testing.assert_close(y.float(), ref.reshape(b, L, -1).float(), rtol=2e-2, atol=2e-2)
+
+
+# ---------------------------------------------------------------------------
+# addresses (CPU)
+# ---------------------------------------------------------------------------
+
+def test_lds_addresses():
+    """Copies and operand reads of a step meet: every byte of B, C, x and W
+    that a lane reads lies inside its buffer and holds the element the
+    product needs."""
+    pin(F, "return (2 * row) & 14;",
+        "const int row = 4 * (DPW * wave + m) + crow;",
+        "(cslot ^ bsw(row & 15))", "(cslot ^ (row & 15))",
+        "boff[nt] = trow * kN + 8 * ((4 * nt + 2 * (g & 1) + (q & 1)) ^ bsw(trow)) + 4 * (q >> 1);",
+        "const int coff = r * kN + 8 * (hl ^ (r & 15));",
+        "cl + (coff ^ (16 * kb)) + 32 * t * kN",
+        "const int xoff = trow * kP + 8 * ((4 * w + 2 * (g & 1) + (q >> 1)) ^ (trow & 7)) + 4 * (q & 1);",
+        "const int q = i & 3, trow = 4 * hl + (i >> 2);",
+        "lds_read_tr(bs + boff[nt] + 16 * kb * kN), lds_read_tr(bs + boff[nt] + (16 * kb + 8) * kN)",
+        "lds_read_tr(xb + xoff + 16 * kb * kP), lds_read_tr(xb + xoff + (16 * kb + 8) * kP)")
+    lane = np.arange(64)
+    hl, r, g, i = lane >> 5, lane & 31, lane >> 4, lane & 15
+    q, trow = i & 3, 4 * hl + (i >> 2)
+    bsw = lambda row: (2 * row) & 14  # noqa: E731
+    # LDS images: [row, column] of each 16-bit slot, as the copies place them
+    img_b, img_c = np.full((64 * 128, 2), -1), np.full((64 * 128, 2), -1)
+    img_x = np.full((64 * 64, 2), -1)
+    for d in range(16):
+        row, slot = 4 * d + (lane >> 4), lane & 15
+        for e in range(8):
+            dst = d * 512 + lane * 8 + e
+            img_b[dst] = np.stack([row, 8 * (slot ^ bsw(row & 15)) + e], 1)
+            img_c[dst] = np.stack([row, 8 * (slot ^ (row & 15)) + e], 1)
+    for blk in range(8):
+        row = 8 * blk + (lane >> 3)
+        for e in range(8):
+            img_x[blk * 512 + lane * 8 + e] = np.stack([row, 8 * ((lane & 7) ^ (lane >> 3)) + e], 1)
+    for img in (img_b, img_c, img_x):
+        assert (img >= 0).all()
+
+    def tr(addr):
+        """element [lane] <- 4 consecutive elements through the transposing read: [64, 4] slots"""
+        out = np.empty((64, 4), np.int64)
+        for k in range(64):
+            base, j = k & 48, k & 15
+            for rr in range(4):
+                out[k, rr] = addr[base + 4 * rr + j // 4] + j % 4
+        return out
+
+    for kb in range(4):
+        tokens = np.stack([16 * kb + 8 * (j // 4) + 4 * hl + j % 4 for j in range(8)], 1)
+        for nt in range(4):
+            a0 = trow * 128 + 8 * ((4 * nt + 2 * (g & 1) + (q & 1)) ^ bsw(trow)) + 4 * (q >> 1)
+            slots = np.concatenate([tr(a0 + 16 * kb * 128), tr(a0 + (16 * kb + 8) * 128)], 1)
+            inside("B", slots, 0, 64 * 128)
+            # row r of the tile is n = 32 nt + 16 (k >> 1) + 8 h + 4 (k & 1) + jj for r = 8 k + 4 h + jj
+            k, h2, jj = r >> 3, (r >> 2) & 1, r & 3
+            n = 32 * nt + 16 * (k >> 1) + 8 * h2 + 4 * (k & 1) + jj
+            assert (img_b[slots][..., 0] == tokens).all() and (img_b[slots][..., 1] == n[:, None]).all()
+        for w in range(2):
+            a0 = trow * 64 + 8 * ((4 * w + 2 * (g & 1) + (q >> 1)) ^ (trow & 7)) + 4 * (q & 1)
+            slots = np.concatenate([tr(a0 + 16 * kb * 64), tr(a0 + (16 * kb + 8) * 64)], 1)
+            inside("x", slots, 0, 64 * 64)
+            assert (img_x[slots][..., 0] == tokens).all() and (img_x[slots][..., 1] == (32 * w + r)[:, None]).all()
+    for kb in range(8):
+        for t in range(2):
+            a0 = ((r * 128 + 8 * (hl ^ (r & 15))) ^ (16 * kb)) + 32 * t * 128
+            slots = a0[:, None] + np.arange(8)
+            inside("C", slots, 0, 64 * 128)
+            assert (img_c[slots][..., 0] == (32 * t + r)[:, None]).all()
+            # S's lane values of K step kb: n = 16 kb + 8 hl + j
+            assert (img_c[slots][..., 1] == (16 * kb + 8 * hl)[:, None] + np.arange(8)).all()
+
+
+def test_w_tiles():
+    """The ten causal tiles, five per wave, fill their halves of W's blocks in
+    the order the diagonal product reads them; the two tiles above the
+    diagonal inside the blocks are the zeroed ones."""
+    pin(F, "constexpr int kT[5] = {0, 2, 1, 2, 2}, kDT[5] = {1, 1, 2, 1, 1};",
+        "constexpr int kS[5] = {0, 2, 0, 0, 1}, kDS[5] = {1, 1, 2, 1, -1};",
+        "constexpr int dS[3] = {1, 2, -1}, dW[3] = {512 + 128, 2048, -512 + 128};",
+        "asoff[k] = 16 * dS[k] * w + 4 * g;", "woff[k] = dW[k] * w + ((g & 1) * 32 + i) * 8 + 4 * (g >> 1);",
+        "if (k < 2) aloff[k] = 16 * dS[k] * w + i;",
+        "constexpr int kDI[5] = {0, 0, 1, 0, 2}, kTI[5] = {0, 0, 1, 0, 0};",
+        "woff[kDI[kb]] + ((t0 >> 1) * 2 + s0) * 512 + (t0 & 1) * 128",
+        "&wl[hh][(w == 0 ? 1 : 5) * 512 + ((g & 1) * 32 + i) * 8 + 4 * (g >> 1)]")
+    kT, kDT, kS, kDS = [0, 2, 1, 2, 2], [1, 1, 2, 1, 1], [0, 2, 0, 0, 1], [1, 1, 2, 1, -1]
+    dS, dW, kDI, kTI = [1, 2, -1], [640, 2048, -384], [0, 0, 1, 0, 2], [0, 0, 1, 0, 0]
+    lane = np.arange(64)
+    g, i = lane >> 4, lane & 15
+    img = np.full((6 * 512, 2), -1)   # (s, l) of each slot of W
+    for w in range(2):
+        zero = (1 if w == 0 else 5) * 512 + ((g & 1) * 32 + i) * 8 + 4 * (g >> 1)
+        for jj in range(4):
+            img[zero + jj] = -2
+    seen = set()
+    for w in range(2):
+        for m in range(5):
+            t, s = kT[m] + kDT[m] * w, kS[m] + kDS[m] * w
+            assert 0 <= s <= t <= 3 and (s == t) == (m < 2)
+            seen.add((t, s))
+            assert (16 * dS[kDI[m]] * w + 4 * g + 16 * kS[m] == 16 * s + 4 * g).all()
+            assert (16 * dS[kTI[m]] * w + i + 16 * kT[m] == 16 * t + i).all()
+            at = dW[kDI[m]] * w + ((g & 1) * 32 + i) * 8 + 4 * (g >> 1) + ((kT[m] >> 1) * 2 + kS[m]) * 512 + (kT[m] & 1) * 128
+            inside("W", at, 0, 6 * 512 - 3)
+            for jj in range(4):
+                assert (img[at + jj] == -1).all()
+                img[at + jj] = np.stack([16 * s + 4 * g + jj, 16 * t + i], 1)
+    assert len(seen) == 10
+    hl, r = lane >> 5, lane & 31
+    for blk, (tile, kb) in enumerate([(0, 0), (0, 1), (1, 0), (1, 1), (1, 2), (1, 3)]):
+        for j in range(8):
+            got = img[blk * 512 + lane * 8 + j]
+            s = 16 * kb + 8 * (j // 4) + 4 * hl + j % 4
+            l = 32 * tile + r  # noqa: E741
+            above = (s // 16) > (l // 16)
+            assert (got[above] == -2).all()
+            assert (got[~above, 0] == s[~above]).all() and (got[~above, 1] == l[~above]).all()

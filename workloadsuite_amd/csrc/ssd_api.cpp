@@ -13,6 +13,7 @@
 
 namespace {
 
+using ssd::ChainScanArgs;
 using ssd::ChunkPrepArgs;
 using ssd::ChunkScanArgs;
 using ssd::ChunkStateArgs;
@@ -399,6 +400,108 @@ int run_core(const ssd_dims* d, int dtype, const CumsumArgs* k1, const void* x, 
   const int sd = f32_layout(state_dtype) ? SSD_DTYPE_F32 : state_dtype;
   if ((rc = run_state_passing(d, dtype, sa, pa, sd, s))) return rc;
   return hip_status(ssd::launch_chunk_scan(ca, dtype, sd, s));
+}
+
+// ---- the core as one walk per chain (ssd_chain_scan.hip) ----
+
+// Its workspace, inside the forward's: Acs and the decays at 64-token steps,
+// chain_prep's operands, the states entering the segments.
+struct ChainWs {
+  size_t acs, decay, cb, ct, cscale, seg, segdec, total;
+};
+
+ChainWs chain_ws(const ssd_dims* d, int dtype, int nseg) {
+  const int64_t steps = d->seqlen / 64, bhs = d->batch * d->nheads * steps, bsg = d->batch * steps * d->ngroups;
+  const bool ct = dtype == SSD_DTYPE_BF16;
+  ChainWs w;
+  w.acs = 0;
+  w.decay = round_up((size_t)bhs * 64 * sizeof(float));
+  w.cb = w.decay + round_up((size_t)bhs * sizeof(float));
+  w.ct = w.cb + round_up(ssd::chain_scan_cb_bytes(bsg));
+  w.cscale = w.ct + (ct ? round_up(ssd::chain_scan_ct_bytes(bsg)) : 0);
+  w.seg = w.cscale + (ct ? round_up(ssd::chain_scan_cscale_bytes(bsg)) : 0);
+  const size_t bhseg = nseg > 1 ? (size_t)(d->batch * d->nheads * nseg) : 0;
+  w.segdec = w.seg + round_up(bhseg * d->headdim * d->dstate * sizeof(float));
+  w.total = w.segdec + round_up(bhseg * sizeof(float));
+  return w;
+}
+
+bool vec_rows(const void* p, const int64_t* strides, int n, int dtype) {
+  return check_vec_operand(p, strides, n, dtype) == SSD_OK;
+}
+
+// The plan of the core of 16-bit inputs with f32 states as a chain walk, or
+// nseg 0 where it does not apply or the stage kernels are the faster way.
+ssd::ChainScanPlan chain_plan(const ssd_dims* d, int dtype, const int64_t x_strides[4], const int64_t b_strides[4],
+                              const int64_t c_strides[4], const int64_t* dt_strides, const void* y,
+                              const int64_t y_strides[4], const ssd_epilogue* epi, size_t ws_bytes) {
+  const ssd::ChainScanPlan none{0, 0, false};
+  if ((dtype != SSD_DTYPE_BF16 && dtype != SSD_DTYPE_F16) || d->dstate != 128 || d->headdim != 64) return none;
+  if (!vec_rows(y, y_strides, 4, dtype)) return none;
+  if (epi && (!epi->z || !dt_strides || !vec_rows(epi->z, epi->z_strides, 4, dtype))) return none;
+  // lane offsets inside a step are 32-bit
+  for (int64_t st : {x_strides[1], b_strides[1], c_strides[1], dt_strides ? dt_strides[1] : 0})
+    if (st > (1 << 23)) return none;
+  const ssd::ChainScanPlan plan = ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, epi != nullptr);
+  if (plan.nseg == 0 || chain_ws(d, dtype, plan.nseg).total > ws_bytes) return none;
+  return plan;
+}
+
+int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan, CumsumArgs k1, const void* x, const int64_t x_strides[4],
+                   const void* bmat, const int64_t b_strides[4], const void* cmat, const int64_t c_strides[4],
+                   const float* dt, const int64_t dt_strides[3], const float* initial_states, void* y,
+                   const int64_t y_strides[4], float* final_states, char* ws, const ssd_epilogue* epi, hipStream_t s) {
+  const ChainWs w = chain_ws(d, dtype, plan.nseg);
+  k1.chunk = 64;
+  k1.nchunks = (int)(d->seqlen / 64);
+  k1.acs = reinterpret_cast<float*>(ws + w.acs);
+  k1.decay = reinterpret_cast<float*>(ws + w.decay);
+  ChainScanArgs p;
+  p.x = x;
+  p.sxb = x_strides[0];
+  p.sxl = x_strides[1];
+  p.sxh = x_strides[2];
+  p.bm = bmat;
+  p.sbb = b_strides[0];
+  p.sbl = b_strides[1];
+  p.sbg = b_strides[2];
+  p.cm = cmat;
+  p.scb = c_strides[0];
+  p.scl = c_strides[1];
+  p.scg = c_strides[2];
+  p.dt = dt;
+  p.sdb = dt ? dt_strides[0] : 0;
+  p.sdl = dt ? dt_strides[1] : 0;
+  p.sdh = dt ? dt_strides[2] : 0;
+  p.acs = k1.acs;
+  p.cb = reinterpret_cast<float*>(ws + w.cb);
+  p.ct = ws + w.ct;
+  p.cscale = reinterpret_cast<float*>(ws + w.cscale);
+  p.init = initial_states;
+  p.final_state = final_states;
+  p.seg_states = reinterpret_cast<float*>(ws + w.seg);
+  p.seg_decay = reinterpret_cast<float*>(ws + w.segdec);
+  p.y = y;
+  p.syb = y_strides[0];
+  p.syl = y_strides[1];
+  p.syh = y_strides[2];
+  if (epi) {
+    p.dskip = epi->D;
+    p.z = epi->z;
+    p.szb = epi->z_strides[0];
+    p.szl = epi->z_strides[1];
+    p.szh = epi->z_strides[2];
+  }
+  p.batch = (int)d->batch;
+  p.nsteps = (int)(d->seqlen / 64);
+  p.nheads = (int)d->nheads;
+  p.ngroups = (int)d->ngroups;
+  p.nseg = plan.nseg;
+  p.seg_len = plan.seg_len;
+  p.wide = plan.wide;
+  int rc;
+  if ((rc = hip_status(ssd::launch_chain_prep(p, k1, dtype, s)))) return rc;
+  return hip_status(ssd::launch_chain_scan(p, dtype, s));
 }
 
 // ---- the layer around the core ----
@@ -819,6 +922,13 @@ int ssd_forward(const ssd_dims* d, int dtype, const void* x, const int64_t x_str
   char* ws = static_cast<char*>(workspace);
   const CumsumArgs k1 = make_cumsum_args(d, a, a_strides, reinterpret_cast<float*>(ws + w.acs),
                                          reinterpret_cast<float*>(ws + w.decay));
+  const ssd::ChainScanPlan plan =
+      state_dtype == SSD_DTYPE_F32
+          ? chain_plan(d, dtype, x_strides, b_strides, c_strides, dt ? dt_strides : nullptr, y, y_strides, nullptr, w.total)
+          : ssd::ChainScanPlan{0, 0, false};
+  if (plan.nseg > 0)
+    return run_chain_scan(d, dtype, plan, k1, x, x_strides, bmat, b_strides, cmat, c_strides, dt, dt_strides, initial_states, y,
+                          y_strides, final_states, ws, nullptr, (hipStream_t)stream);
   return run_core(d, dtype, &k1, x, x_strides, bmat, b_strides, cmat, c_strides, dt, dt_strides, initial_states, y,
                   y_strides, final_states, ws, w, state_dtype, nullptr, (hipStream_t)stream);
 }
@@ -955,6 +1065,10 @@ int ssd_layer_forward(const ssd_dims* d, int dtype, const ssd_layer_params* prm,
   epi.z_strides[1] = z_strides[1];
   epi.z_strides[2] = P * z_strides[2];
   epi.z_strides[3] = z_strides[2];
+  const ssd::ChainScanPlan plan = chain_plan(d, dtype, xs4, b_strides, c_strides, dts, y, ys4, &epi, w.cw.total);
+  if (plan.nseg > 0)
+    return run_chain_scan(d, dtype, plan, k1, x_out, xs4, bmat, b_strides, cmat, c_strides, dt_out, dts, nullptr, y, ys4,
+                          nullptr, core, &epi, s);
   return run_core(d, dtype, &k1, x_out, xs4, bmat, b_strides, cmat, c_strides, dt_out, dts, nullptr, y, ys4,
                   nullptr, core, w.cw, SSD_DTYPE_F32, &epi, s);
 }

@@ -214,6 +214,47 @@ hipError_t launch_chunk_scan_f32(const ChunkScanArgs& a, hipStream_t stream);
 bool chunk_scan_b16_supported(const ChunkScanArgs& a, int dtype, int state_dtype);
 hipError_t launch_chunk_scan_b16(const ChunkScanArgs& a, int dtype, hipStream_t stream);
 
+// The core of 16-bit inputs at d_state 128 as one walk per (b, h) chain, 64
+// tokens per step with the state in registers (ssd_chain_scan.hip).
+struct ChainScanArgs {
+  const void* x;
+  int64_t sxb, sxl, sxh;  // x [b, L, h, P], unit stride over P
+  const void* bm;
+  int64_t sbb, sbl, sbg;  // bmat, cmat [b, L, g, N], unit stride over N
+  const void* cm;
+  int64_t scb, scl, scg;
+  const float* dt;        // optional [b, L, h]
+  int64_t sdb, sdl, sdh;
+  const float* acs;       // [b, h, steps, 64] (K1 at chunk 64)
+  float* cb;              // chain_prep: C.B^T tiles per (b, step, group)
+  void* ct;               // chain_prep, bf16 inputs: C as f16 rows
+  float* cscale;          // ... and their scales
+  const float* init;      // optional [b, h, P, N]
+  float* final_state;     // optional [b, h, P, N]
+  float* seg_states;      // nseg > 1: the state entering each segment [b, nseg, h, P, N]
+  float* seg_decay;       // ... and the segments' decays [b, h, nseg]
+  void* y;
+  int64_t syb, syl, syh;  // y [b, L, h, P], 16-byte aligned rows
+  const float* dskip = nullptr;  // epilogue (with z): y = (y + dskip[h] x) * silu(z)
+  const void* z = nullptr;       // [b, L, h, P], 16-byte aligned rows
+  int64_t szb = 0, szl = 0, szh = 0;
+  int batch, nsteps, nheads, ngroups, nseg, seg_len;
+  bool wide = false;      // epilogue: four heads per workgroup instead of two
+};
+// How the chains of a shape are cut: nseg segments of seg_len steps; nseg 0:
+// not supported, or the stage kernels are as fast.
+struct ChainScanPlan {
+  int nseg, seg_len;
+  bool wide;
+};
+ChainScanPlan chain_scan_plan(int64_t batch, int64_t steps, int64_t nheads, int64_t ngroups, bool epi);
+// bytes of cb / ct / cscale for `steps` = batch * nsteps * ngroups
+size_t chain_scan_cb_bytes(int64_t steps);
+size_t chain_scan_ct_bytes(int64_t steps);
+size_t chain_scan_cscale_bytes(int64_t steps);
+hipError_t launch_chain_prep(const ChainScanArgs& a, const CumsumArgs& ca, int dtype, hipStream_t stream);
+hipError_t launch_chain_scan(const ChainScanArgs& a, int dtype, hipStream_t stream);
+
 // The whole forward in one launch for small states and short chains
 // (ssd_small.hip): d_state 16 / 32, chunk 64 / 128, at most kSmallMaxChunks
 // chunks per chain, f32 states kept in LDS; one workgroup per (b, h) chain.

@@ -308,9 +308,13 @@ def ssd_forward(X, A, B, C, chunk_size, dt=None, initial_states=None,
     float32.  ``state_format`` (float32 states, 16-bit inputs): how the states
     entering each chunk reach chunk_scan --
 
-    * None (the default): f16 rows with a power-of-two scale per row
-      ("f16s") wherever a 16-bit chunk_scan reads them: chunk 256 with
-      d_state 64 / 128, and chunk 64 / 128 with chunk x d_state <= 8192.
+    * None (the default): the library's choice.  At d_state 128 with an even
+      number of heads per group and enough work for the GPU the whole core
+      runs as a walk along the (batch, head) chains with the state in float32
+      registers, and no states are handed over at all.  Otherwise f16 rows
+      with a power-of-two scale per row ("f16s") wherever a 16-bit chunk_scan
+      reads them: chunk 256 with d_state 64 / 128, and chunk 64 / 128 with
+      chunk x d_state <= 8192.
       Where chunk_state and state_passing then run as two launches (chunk 256
       outside the one-launch state chain, and the chain's segments) the local
       states between them cross HBM as f16 rows with a scale per row and
@@ -321,7 +325,7 @@ def ssd_forward(X, A, B, C, chunk_size, dt=None, initial_states=None,
       state within ~1e-3 of its scale).
     * "split": hi/lo pairs of the inputs' type at chunk 256 (plain float32
       at chunk 64 / 128); every local state stays float32.
-    * "f16s": as the default.
+    * "f16s": f16 rows as above, never the walk.
     """
     key = (_layout_key(X), _layout_key(A), _layout_key(B), _layout_key(C), _layout_key(dt),
            _layout_key(initial_states), chunk_size, return_final_states, state_dtype, state_format)
