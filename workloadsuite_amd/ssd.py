@@ -677,11 +677,54 @@ def chunk_scan(X, B, C, Acs, states, dt=None, prep=None, split=False, D=None, z=
     return Y
 
 
+# decode_step's and ssd_layer's per-call host work, kept per layout as
+# ssd_forward's is (_PLANS): for operands the kernels take as they are.  Nothing
+# of a call's own is kept: pointers go into structs made for the call.
+_DECODE_PLANS = {}
+_LAYER_PLANS = {}
+
+
+class _DecodePlan(NamedTuple):
+    dims: object
+    dtype: int
+    strides: tuple     # x, B, C, a (and dt), y
+    z_strides: object  # or None
+    y_shape: tuple
+
+
+class _LayerPlan(NamedTuple):
+    dims: object
+    dtype: int
+    width: int         # conv kernel width
+    strides: tuple     # x, z, B, C, dt, y
+    nbytes: int
+
+
 def decode_step(state, x, B, C, a, dt=None, D=None, z=None):
     """One token of the recurrence, in place on ``state`` [b, h, P, N] f32
     (e.g. ssd_forward's final state): state = exp(a) state + dt x B^T, then
     y = state C (+ D x, * silu(z)).  x, z [b, h, P]; B, C [b, g, N] of x's
     dtype; a, dt [b, h] f32 (dt None means 1).  Returns y [b, h, P]."""
+    key = (_layout_key(state), _layout_key(x), _layout_key(B), _layout_key(C), _layout_key(a), _layout_key(dt),
+           _layout_key(D), _layout_key(z))
+    plan = _DECODE_PLANS.get(key)
+    if plan is None or not _aligned(state, a, dt, D):
+        return _decode_step(state, x, B, C, a, dt, D, z, key)
+    dev = x.device
+    y = torch.empty(plan.y_shape, dtype=x.dtype, device=dev)
+    sx, sb, sc, sad, sy = plan.strides
+    epi = None
+    if plan.z_strides is not None:
+        epi = ctypes.byref(_lib.SSDEpilogue(0 if D is None else D.data_ptr(), 0 if z is None else z.data_ptr(),
+                                            plan.z_strides))
+    _lib.check(_lib.load().ssd_decode_step(
+        ctypes.byref(plan.dims), plan.dtype, state.data_ptr(), x.data_ptr(), sx, B.data_ptr(), sb, C.data_ptr(), sc,
+        a.data_ptr(), None if dt is None else dt.data_ptr(), sad, y.data_ptr(), sy, epi, _stream_fast(dev)))
+    return y
+
+
+def _decode_step(state, x, B, C, a, dt, D, z, key):
+    """The checks, operand conversions and call of decode_step (and its plan for the layout)."""
     if state.dim() != 4 or state.dtype != torch.float32:
         raise ValueError("state must be [b, h, P, N] float32")
     b, h, P, N = state.shape
@@ -700,6 +743,7 @@ def decode_step(state, x, B, C, a, dt=None, D=None, z=None):
     if D is not None and D.numel() != h:
         raise ValueError(f"D must have {h} elements")
     d = _lib.dims(b, 1, h, P, N, g, 1)
+    given = (x, B, C, a, dt, D, z)
     x, Bm, Cm = _rows3(x), _rows3(B), _rows3(C)
     a = _f32_contig(a)
     dt = _f32_contig(dt)
@@ -721,10 +765,18 @@ def decode_step(state, x, B, C, a, dt=None, D=None, z=None):
             keep.append(z)
         _keep = keep
     st2 = lambda t: (ctypes.c_int64 * 2)(t.stride(0), t.stride(1))  # noqa: E731
+    strides = (st2(x), st2(Bm), st2(Cm), st2(a), st2(y))
     _lib.check(_lib.load().ssd_decode_step(
-        ctypes.byref(d), _DTYPES[x.dtype], _ptr(state), _ptr(x), st2(x), _ptr(Bm), st2(Bm), _ptr(Cm), st2(Cm),
-        _ptr(a), _ptr(dt), st2(a), _ptr(y), st2(y), ctypes.byref(epi) if epi is not None else None, _stream(dev)))
+        ctypes.byref(d), _DTYPES[x.dtype], _ptr(state), _ptr(x), strides[0], _ptr(Bm), strides[1], _ptr(Cm), strides[2],
+        _ptr(a), _ptr(dt), strides[3], _ptr(y), strides[4], ctypes.byref(epi) if epi is not None else None, _stream(dev)))
     del _keep
+    # the same layout next time, where nothing was copied or converted (D, of
+    # any shape with h elements in a row, is read as its h floats)
+    x0, B0, C0, a0, dt0, D0, z0 = given
+    if (all(_unchanged(t, t0) for t, t0 in ((x, x0), (Bm, B0), (Cm, C0), (a, a0), (dt, dt0), (z, z0)))
+            and (D0 is None or (D.data_ptr() == D0.data_ptr() and D0.dtype == torch.float32))
+            and len(_DECODE_PLANS) < _PLANS_MAX):
+        _DECODE_PLANS[key] = _DecodePlan(d, _DTYPES[x.dtype], strides, None if epi is None else epi.z_strides, (b, h, P))
     return y
 
 
@@ -796,6 +848,26 @@ def ssd_layer(x, z, B, C, dt, conv_weight, conv_bias, dt_bias, A_log, D, chunk_s
     [h*P, 1, k], ``conv_bias`` [h*P] or None, ``dt_bias`` [h], ``A_log`` [h],
     ``D`` [h] or None: MR's parameters.  Returns y [b, L, h*P] in x's dtype,
     out_proj's input."""
+    key = (_layout_key(x), _layout_key(z), _layout_key(B), _layout_key(C), _layout_key(dt), _layout_key(conv_weight),
+           _layout_key(conv_bias), _layout_key(dt_bias), _layout_key(A_log), _layout_key(D), chunk_size, nheads)
+    plan = _LAYER_PLANS.get(key)
+    if plan is None or not _aligned(B, C, A_log):
+        return _ssd_layer(x, z, B, C, dt, conv_weight, conv_bias, dt_bias, A_log, D, chunk_size, nheads, key)
+    dev = x.device
+    Dv = None if D is None else _f32_contig(D)
+    prm = _lib.SSDLayerParams(plan.width, conv_weight.data_ptr(), 0 if conv_bias is None else conv_bias.data_ptr(),
+                              dt_bias.data_ptr(), A_log.data_ptr(), 0 if Dv is None else Dv.data_ptr())
+    sx, sz, sb, sc, sdt, sy = plan.strides
+    ws = torch.empty(max(plan.nbytes, 1), dtype=torch.uint8, device=dev)
+    y = torch.empty(x.shape, dtype=x.dtype, device=dev)
+    _lib.check(_lib.load().ssd_layer_forward(
+        ctypes.byref(plan.dims), plan.dtype, ctypes.byref(prm), x.data_ptr(), sx, z.data_ptr(), sz, B.data_ptr(), sb,
+        C.data_ptr(), sc, dt.data_ptr(), sdt, y.data_ptr(), sy, ws.data_ptr(), plan.nbytes, _stream_fast(dev)))
+    return y
+
+
+def _ssd_layer(x, z, B, C, dt, conv_weight, conv_bias, dt_bias, A_log, D, chunk_size, nheads, key):
+    """The checks, operand conversions and call of ssd_layer (and its plan for the layout)."""
     b, L, d_inner = x.shape
     if z.shape != x.shape or dt.shape != (b, L, nheads) or d_inner % nheads != 0:
         raise ValueError("x and z must be [b, L, h*P] and dt [b, L, h]")
@@ -812,15 +884,24 @@ def ssd_layer(x, z, B, C, dt, conv_weight, conv_bias, dt_bias, A_log, D, chunk_s
         raise ValueError("x, z, B, C and dt must share a supported dtype")
     dev = _device_check(x, z, B, C, dt, conv_weight, dt_bias, A_log)
     d = _dims(b, L, nheads, P, N, g, chunk_size)
-    prm, _keep = _layer_params(conv_weight, conv_bias, dt_bias, A_log, D, d_inner, nheads, dtype, dev)
+    prm, keep = _layer_params(conv_weight, conv_bias, dt_bias, A_log, D, d_inner, nheads, dtype, dev)
+    given = (x, z, dt, B, C)
     x, z, dt = _rows3(x), _rows3(z), _rows3(dt)
     Bm, Cm = _vec_operand(B.detach()), _vec_operand(C.detach())
     lib = _lib.load()
     nbytes = lib.ssd_layer_workspace_bytes(ctypes.byref(d), _DTYPES[dtype])
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     y = torch.empty((b, L, d_inner), dtype=dtype, device=dev)
+    strides = tuple(_lib.strides(t) for t in (x, z, Bm, Cm, dt, y))
     _lib.check(lib.ssd_layer_forward(
-        ctypes.byref(d), _DTYPES[dtype], ctypes.byref(prm), _ptr(x), _lib.strides(x), _ptr(z), _lib.strides(z),
-        _ptr(Bm), _lib.strides(Bm), _ptr(Cm), _lib.strides(Cm), _ptr(dt), _lib.strides(dt), _ptr(y),
-        _lib.strides(y), _ptr(ws), nbytes, _stream(dev)))
+        ctypes.byref(d), _DTYPES[dtype], ctypes.byref(prm), _ptr(x), strides[0], _ptr(z), strides[1],
+        _ptr(Bm), strides[2], _ptr(Cm), strides[3], _ptr(dt), strides[4], _ptr(y), strides[5], _ptr(ws), nbytes,
+        _stream(dev)))
+    # the same layout next time, where nothing but D was copied or converted
+    w, bias, dtb, alog, _ = keep
+    as_is = (all(_unchanged(t, t0) for t, t0 in zip((x, z, dt, Bm, Cm), given))
+             and all((t is None and t0 is None) or (t.data_ptr() == t0.data_ptr() and t.dtype == t0.dtype)
+                     for t, t0 in ((w, conv_weight), (bias, conv_bias), (dtb, dt_bias), (alog, A_log))))
+    if as_is and len(_LAYER_PLANS) < _PLANS_MAX:
+        _LAYER_PLANS[key] = _LayerPlan(d, _DTYPES[dtype], conv_weight.shape[-1], strides, nbytes)
     return y
