@@ -264,7 +264,9 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * (operands, then for few chains the end states of their segments, then the
  * walk: two to four launches; the workspace is the same).  Its results differ
  * from the stage kernels' by rounding; SSD_STATE_F16S (or SPLIT) as
- * state_dtype keeps the stage kernels.  Otherwise, all on `stream`: at chunk 256
+ * state_dtype keeps the stage kernels.  f32 inputs at dstate 64 / 128 walk too
+ * (two launches) with an even number of heads per group and more than two
+ * chains per CU.  Otherwise, all on `stream`: at chunk 256
  * with 16-bit inputs K1 + K0 as one launch, then K2 + K3 as one state-chain
  * launch (the chain's mixed plan adds K3 over the chains it leaves as
  * segments) or K2 then K3 where the chains are too few, then K4: three or

@@ -202,9 +202,9 @@ def test_w_tiles():
     """The ten causal tiles, five per wave, fill their halves of W's blocks in
     the order the diagonal product reads them; the two tiles above the
     diagonal inside the blocks are the zeroed ones."""
-    pin(F, "constexpr int kT[5] = {0, 2, 1, 2, 2}, kDT[5] = {1, 1, 2, 1, 1};",
-        "constexpr int kS[5] = {0, 2, 0, 0, 1}, kDS[5] = {1, 1, 2, 1, -1};",
-        "constexpr int dS[3] = {1, 2, -1}, dW[3] = {512 + 128, 2048, -512 + 128};",
+    pin("ssd_chain_step.h", "constexpr int kT[5] = {0, 2, 1, 2, 2}, kDT[5] = {1, 1, 2, 1, 1};",
+        "constexpr int kS[5] = {0, 2, 0, 0, 1}, kDS[5] = {1, 1, 2, 1, -1};")
+    pin(F, "constexpr int dS[3] = {1, 2, -1}, dW[3] = {512 + 128, 2048, -512 + 128};",
         "asoff[k] = 16 * dS[k] * w + 4 * g;", "woff[k] = dW[k] * w + ((g & 1) * 32 + i) * 8 + 4 * (g >> 1);",
         "if (k < 2) aloff[k] = 16 * dS[k] * w + i;",
         "constexpr int kDI[5] = {0, 0, 1, 0, 2}, kTI[5] = {0, 0, 1, 0, 0};",

@@ -1,0 +1,155 @@
+"""The chain walk of f32 inputs (csrc/ssd_chain_scan_f32.hip): ssd_forward at
+d_state 64 / 128 with more than one workgroup (two chains of a group) per CU.
+
+GPU: against the float64 oracle (chunked evaluation at 64), y and the final state to
+the f32 tolerance of the parity tests (rtol = atol = 1e-4: sums of up to 64 +
+d_state f32 products of order-1 terms).
+
+CPU: the per-lane addresses of the copies and operand reads, and the C.B^T tiles a
+lane takes, restated and pinned to the source."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ssd_oracle as O
+from test_address_bounds import inside, pin
+from workloadsuite_amd import ssd as S
+
+DEV = "cuda"
+F = "ssd_chain_scan_f32.hip"
+
+# b, L, h, g, N, chunk: just over one workgroup per CU; one step; an odd number of
+# steps; two heads per group; chunk 128
+SHAPES = [
+    (9, 192, 64, 4, 64, 64),
+    (40, 64, 24, 1, 64, 64),
+    (9, 320, 64, 32, 128, 64),
+    (17, 256, 32, 1, 128, 128),
+    (20, 384, 48, 8, 64, 128),
+]
+
+
+def case(b, L, h, g, N, seed):
+    gen = torch.Generator().manual_seed(seed)
+    X = torch.randn(b, L, h, 64, generator=gen)
+    A = -torch.rand(b, L, h, generator=gen) * 0.3
+    B = torch.randn(b, L, g, N, generator=gen) * N ** -0.5
+    C = torch.randn(b, L, g, N, generator=gen) * N ** -0.5
+    dt = torch.rand(b, L, h, generator=gen) + 0.1
+    init = torch.randn(b, h, 64, N, generator=gen)
+    return X, A, B, C, dt, init
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,L,h,g,N,chunk", SHAPES)
+@pytest.mark.parametrize("opts", [True, False])
+def test_forward(b, L, h, g, N, chunk, opts):
+    print("CASE f32 chain walk", b, L, h, g, N, chunk, opts, flush=True)
+    X, A, B, C, dt, init = case(b, L, h, g, N, seed=L + h)
+    dt, init = (dt, init) if opts else (None, None)
+    hs = [0, 1, h // 2, h - 1]
+    grp = [k // (h // g) for k in hs]
+    ref, fref = O.ssd_chunked(X[:, :, hs], A[:, :, hs], B[:, :, grp], C[:, :, grp], 64,
+                              dt=None if dt is None else dt[:, :, hs], initial_states=None if init is None else init[:, hs])
+    d = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    Y, final = S.ssd_forward(d(X), d(A), d(B), d(C), chunk, dt=d(dt), initial_states=d(init), return_final_states=True)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(Y[:, :, hs].double().cpu(), ref, rtol=1e-4, atol=1e-4)
+    torch.testing.assert_close(final[:, hs].double().cpu(), fref, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [64, 128])
+def test_strided_operands_match_contiguous_ones(N):
+    """x, B, C and dt as slices of wider tensors, A transposed: the bits of the contiguous call."""
+    print("CASE f32 chain walk, strides", N, flush=True)
+    b, L, h, g = 9, 256, 64, 8
+    X, A, B, C, dt, init = (t.to(DEV) for t in case(b, L, h, g, N, seed=3))
+    wide = torch.zeros(b, L, h * 64 + 2 * g * N + h + 12, device=DEV)
+    at = [4, 4 + h * 64, 4 + h * 64 + g * N, 4 + h * 64 + 2 * g * N]
+    xs, bs, cs = wide[..., at[0]:at[1]], wide[..., at[1]:at[2]], wide[..., at[2]:at[3]]
+    dts = wide[..., at[3]:at[3] + h]
+    xs.copy_(X.flatten(2)), bs.copy_(B.flatten(2)), cs.copy_(C.flatten(2)), dts.copy_(dt)
+    At = A.transpose(1, 2).contiguous().transpose(1, 2)
+    Y0, f0 = S.ssd_forward(X, A, B, C, 64, dt=dt, initial_states=init, return_final_states=True)
+    Y1, f1 = S.ssd_forward(xs.unflatten(2, (h, 64)), At, bs.unflatten(2, (g, N)), cs.unflatten(2, (g, N)), 64, dt=dts,
+                           initial_states=init, return_final_states=True)
+    torch.cuda.synchronize()
+    assert torch.equal(Y0, Y1) and torch.equal(f0, f1)
+
+
+# ---------------------------------------------------------------------------
+# addresses (CPU)
+# ---------------------------------------------------------------------------
+
+@pytest.mark.parametrize("N", [64, 128])
+def test_lds_addresses(N):
+    """Copies and operand reads meet: the element a lane reads lies inside its
+    buffer and is the one its K slot stands for."""
+    pin(F, "const int row0 = RPB * wave + lane / PPR, slot = lane % PPR;",
+        "4 * (slot ^ (8 * ((row0 >> 2) & 1)))", "4 * (slot ^ (row0 & 15))", "4 * (slot ^ ((row0 + RPB * kWaves) & 15))",
+        "const int coff = r * PPR + (hl ^ (r & 15));", "[(co ^ (2 * kk)) + 32 * t * PPR]",
+        "const int boff[2] = {4 * hl * N + r + 32 * hl, 4 * hl * N + r - 32 * hl};",
+        "bs[boff[nt & 1] + (8 * kk + jj) * N + 32 * nt]")
+    ppr = N // 4
+    rpb, dpw = 64 // ppr, N // 16
+    lane = np.arange(64)
+    hl, r = lane >> 5, lane & 31
+    img_b, img_c = np.full((64 * N, 2), -1), np.full((64 * N, 2), -1)
+    for wave in range(4):
+        row0, slot = rpb * wave + lane // ppr, lane % ppr
+        for m in range(dpw):
+            row = row0 + 4 * rpb * m
+            pb = slot ^ (8 * ((row0 >> 2) & 1))
+            pc = slot ^ ((row0 + (4 * rpb if m & 1 else 0)) & 15)
+            for e in range(4):
+                dst = (wave + 4 * m) * 256 + lane * 4 + e
+                img_b[dst] = np.stack([row, 4 * pb + e], 1)
+                img_c[dst] = np.stack([row, 4 * pc + e], 1)
+    assert (img_b >= 0).all() and (img_c >= 0).all()
+    for kk in range(N // 8):
+        for t in range(2):
+            piece = ((r * ppr + (hl ^ (r & 15))) ^ (2 * kk)) + 32 * t * ppr
+            for jj in range(4):
+                inside("C", 4 * piece + jj, 0, 64 * N)
+                got = img_c[4 * piece + jj]
+                # the lane's state register kk, jj holds n = 8 kk + 4 hl + jj
+                assert (got[:, 0] == 32 * t + r).all() and (got[:, 1] == 8 * kk + 4 * hl + jj).all()
+    for kk in range(8):
+        for nt in range(N // 32):
+            for jj in range(4):
+                at = 4 * hl * N + r + (-32 if nt & 1 else 32) * hl + (8 * kk + jj) * N + 32 * nt
+                inside("B", at, 0, 64 * N)
+                got = img_b[at]
+                assert (got[:, 0] == 8 * kk + 4 * hl + jj).all() and (got[:, 1] == 32 * nt + r).all()
+
+
+def test_cb_tiles():
+    """The C.B^T values a lane loads are those of its W: rows s of its K slots, column l."""
+    pin(F, "cbv[0][0] = lo + (t1 ? 4 : 0) * 1024, cbv[0][1] = lo + (t1 ? 1 : 0) * 1024;",
+        "cbv[1][0] = lo + (t1 ? 9 : 6) * 1024, cbv[1][1] = lo + (t1 ? 7 : 8) * 1024;",
+        "cbv[2][0] = lo + (t1 ? 5 : 2) * 1024, cbv[2][1] = lo + (t1 ? 3 : 2) * 1024;",
+        "const uint32_t lo = (uint32_t)(hl * 16 + i) * 16;", "cbv[q][k >> 1] + 512 * (k & 1)",
+        "kBlk[12] = {0, 1, 0, 1, 0, 1, 0, 1, 2, 2, 2, 2}, kGrp[12] = {0, 0, 1, 1, 2, 2, 3, 3, 0, 1, 2, 3};")
+    kT, kDT, kS, kDS = [0, 2, 1, 2, 2], [1, 1, 2, 1, 1], [0, 2, 0, 0, 1], [1, 1, 2, 1, -1]
+    img = np.full((10 * 64 * 4, 2), -1)   # (s, l) of each f32 of a step's tiles
+    lane = np.arange(64)
+    for k in range(10):
+        m, w = k >> 1, k & 1
+        t, s = kT[m] + kDT[m] * w, kS[m] + kDS[m] * w
+        for jj in range(4):
+            img[(k * 64 + lane) * 4 + jj] = np.stack([16 * s + 4 * (lane >> 4) + jj, 16 * t + (lane & 15)], 1)
+    hl, r, i = lane >> 5, lane & 31, lane & 15
+    t1 = r >= 16
+    tiles = [[(4, 0), (1, 0)], [(9, 6), (7, 8)], [(5, 2), (3, 2)]]
+    blk, grp = [0, 1, 0, 1, 0, 1, 0, 1, 2, 2, 2, 2], [0, 0, 1, 1, 2, 2, 3, 3, 0, 1, 2, 3]
+    assert sorted(zip(blk, grp)) == [(q, k) for q in range(3) for k in range(4)]
+    for q, k in zip(blk, grp):
+        off = (hl * 16 + i) * 16 + np.where(t1, *tiles[q][k >> 1]) * 1024 + 512 * (k & 1)
+        for jj in range(4):
+            at = off // 4 + jj
+            inside("C.B^T", at, 0, 10 * 64 * 4)
+            s, l = 32 * (q > 1) + 8 * k + 4 * hl + jj, 32 * (q > 0) + r  # noqa: E741
+            kept = s <= l   # above the diagonal the value is masked
+            assert (img[at][kept, 0] == s[kept]).all() and (img[at][kept, 1] == l[kept]).all()

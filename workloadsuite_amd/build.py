@@ -38,7 +38,7 @@ SOURCES = [
     "ssd_decode.hip",
     "ssd_noalloc.hip",
     "ssd_small.hip",
-    "ssd_chain_scan.hip",
+    "ssd_chain_scan.hip", "ssd_chain_scan_f32.hip",
 ]
 
 # The streaming probe behind bench.py --hbm-probe: its own library, outside

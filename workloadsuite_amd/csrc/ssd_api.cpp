@@ -402,7 +402,7 @@ int run_core(const ssd_dims* d, int dtype, const CumsumArgs* k1, const void* x, 
   return hip_status(ssd::launch_chunk_scan(ca, dtype, sd, s));
 }
 
-// ---- the core as one walk per chain (ssd_chain_scan.hip) ----
+// ---- the core as one walk per chain (ssd_chain_scan.hip, ssd_chain_scan_f32.hip) ----
 
 // Its workspace, inside the forward's: Acs and the decays at 64-token steps,
 // chain_prep's operands, the states entering the segments.
@@ -430,19 +430,24 @@ bool vec_rows(const void* p, const int64_t* strides, int n, int dtype) {
   return check_vec_operand(p, strides, n, dtype) == SSD_OK;
 }
 
-// The plan of the core of 16-bit inputs with f32 states as a chain walk, or
-// nseg 0 where it does not apply or the stage kernels are the faster way.
+// The plan of the core with f32 states as a chain walk (16-bit inputs at
+// d_state 128, f32 ones at 64 / 128), or nseg 0 where it does not apply or the
+// stage kernels are the faster way.
 ssd::ChainScanPlan chain_plan(const ssd_dims* d, int dtype, const int64_t x_strides[4], const int64_t b_strides[4],
                               const int64_t c_strides[4], const int64_t* dt_strides, const void* y,
                               const int64_t y_strides[4], const ssd_epilogue* epi, size_t ws_bytes) {
   const ssd::ChainScanPlan none{0, 0, false};
-  if ((dtype != SSD_DTYPE_BF16 && dtype != SSD_DTYPE_F16) || d->dstate != 128 || d->headdim != 64) return none;
+  const bool f32 = dtype == SSD_DTYPE_F32;
+  if ((f32 && epi) || d->headdim != 64 || (f32 ? d->dstate != 64 && d->dstate != 128 : d->dstate != 128)) return none;
   if (!vec_rows(y, y_strides, 4, dtype)) return none;
   if (epi && (!epi->z || !dt_strides || !vec_rows(epi->z, epi->z_strides, 4, dtype))) return none;
   // lane offsets inside a step are 32-bit
   for (int64_t st : {x_strides[1], b_strides[1], c_strides[1], dt_strides ? dt_strides[1] : 0})
     if (st > (1 << 23)) return none;
-  const ssd::ChainScanPlan plan = ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, epi != nullptr);
+  if (f32 && y_strides[1] > (1 << 23)) return none;
+  const ssd::ChainScanPlan plan =
+      f32 ? ssd::chain_scan_f32_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, d->dstate)
+          : ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, epi != nullptr);
   if (plan.nseg == 0 || chain_ws(d, dtype, plan.nseg).total > ws_bytes) return none;
   return plan;
 }
@@ -499,9 +504,11 @@ int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan,
   p.nseg = plan.nseg;
   p.seg_len = plan.seg_len;
   p.wide = plan.wide;
+  const int n = (int)d->dstate;
+  const bool f32 = dtype == SSD_DTYPE_F32;
   int rc;
-  if ((rc = hip_status(ssd::launch_chain_prep(p, k1, dtype, s)))) return rc;
-  return hip_status(ssd::launch_chain_scan(p, dtype, s));
+  if ((rc = hip_status(f32 ? ssd::launch_chain_prep_f32(p, k1, n, s) : ssd::launch_chain_prep(p, k1, dtype, s)))) return rc;
+  return hip_status(f32 ? ssd::launch_chain_scan_f32(p, n, s) : ssd::launch_chain_scan(p, dtype, s));
 }
 
 // ---- the layer around the core ----

@@ -46,132 +46,21 @@
 // Slower: two 16-row halves per wave on 16x16x32 MFMAs (twice the LDS reads: 437
 // against 387 us for the layer span), the MFMAs of a step behind all its copies
 // (a copy stalls its wave while others queue: 6% of a step).
-#include "ssd_cumsum_body.h"
-#include "ssd_device.h"
-#include "ssd_launch.h"
+#include "ssd_chain_step.h"
 #include "../../include/ssd.h"
 
 namespace ssd {
 
 namespace {
 
-constexpr int kQ = 64;       // tokens per step
+constexpr int kQ = kStep;    // tokens per step
 constexpr int kP = 64;       // head dim
 constexpr int kN = 128;      // d_state
-constexpr int kTiles = 10;   // causal 16 x 16 tiles of C.B^T
 // Up to this many segments, each workgroup of the scan forms its entering
 // state itself from the end states of the segments before it (as many reads as
 // state_passing's, no writes and one launch less); above, state_passing does.
 constexpr int kFoldSegs = 4;
 constexpr int kWBlocks = 6;  // 32 (s) x 16 (l) blocks of W
-
-// The causal tiles (row tile t of l, column tile s of s, s <= t) in pairs 2 m +
-// w, one for each wave of a head: (t, s) = (kT[m] + kDT[m] w, kS[m] + kDS[m] w).
-// Pairs 0 and 1 are the diagonal ones.
-constexpr int kT[5] = {0, 2, 1, 2, 2}, kDT[5] = {1, 1, 2, 1, 1};
-constexpr int kS[5] = {0, 2, 0, 0, 1}, kDS[5] = {1, 1, 2, 1, -1};
-
-// C.B^T tiles and, for bf16, the f16 C rows of (batch, step, group) bcg; 4 waves, wave t = row tile t.
-template <typename T>
-__device__ __forceinline__ void chain_prep_body(const ChainScanArgs& p, int bcg, int tid) {
-  const int lane = tid & 63, t = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, i = lane & 15;
-  const int grp = bcg % p.ngroups, bc = bcg / p.ngroups;
-  const int c = bc % p.nsteps, b = bc / p.nsteps;
-  const T* bg = reinterpret_cast<const T*>(p.bm) + (int64_t)b * p.sbb + (int64_t)c * kQ * p.sbl + (int64_t)grp * p.sbg;
-  const T* cg = reinterpret_cast<const T*>(p.cm) + (int64_t)b * p.scb + (int64_t)c * kQ * p.scl + (int64_t)grp * p.scg;
-  frag8<T> cf[4];
-#pragma unroll
-  for (int kc = 0; kc < 4; ++kc) cf[kc] = load8<T>(cg + (int64_t)(16 * t + i) * p.scl + 32 * kc + 8 * g);
-  f32x4* cb = reinterpret_cast<f32x4*>(p.cb) + (int64_t)bcg * kTiles * 64 + lane;
-#pragma unroll
-  for (int k = 0; k < kTiles; ++k) {
-    const int m = k >> 1, wk = k & 1, s = kS[m] + kDS[m] * wk;
-    if (kT[m] + kDT[m] * wk != t) continue;  // wave-uniform
-    f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) d = mma(load8<T>(bg + (int64_t)(16 * s + i) * p.sbl + 32 * kc + 8 * g), cf[kc], d);
-    cb[k * 64] = d;
-  }
-  if constexpr (!std::is_same<T, f16>::value) {
-    // each row as f16 times 2^-e, its largest element in [2^14, 2^15) (bf16
-    // values then convert exactly down to 2^-24 of it), in operand order:
-    // piece 4 kc + g holds n = 32 kc + 4 g .. + 3 and 32 kc + 16 + 4 g .. + 3
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    uint32_t mb = 0;
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-      const auto w = __builtin_bit_cast(u32x4, cf[kc]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) mb = max(mb, max(w[j] & 0x7fffu, (w[j] >> 16) & 0x7fffu));
-    }
-    float m = __uint_as_float(min(mb, 0x7f80u) << 16);  // a NaN counts as inf, as in every lane
-    m = nn_max(m, __shfl_xor(m, 16));
-    m = nn_max(m, __shfl_xor(m, 32));
-    const int e = m > 0.f ? min(max(__builtin_amdgcn_frexp_expf(m) - 15, -100), 100) : 0;
-    f16* row = reinterpret_cast<f16*>(p.ct) + ((int64_t)bcg * kQ + 16 * t + i) * kN;
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-      f16x8 hv;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) hv[j] = (f16)__builtin_ldexpf(to_f32<T>(cf[kc][j]), -e);
-      store8<f16>(row + 32 * kc + 8 * g, hv);
-    }
-    if (g == 0) p.cscale[(int64_t)bcg * kQ + 16 * t + i] = __builtin_ldexpf(1.f, e);
-  }
-}
-
-// K1's blocks (64-token cumsums, 256 threads each) and the prep blocks in one launch.
-template <typename T, typename R, bool RAW>
-__global__ __launch_bounds__(256) void chain_prep_kernel(ChainScanArgs p, CumsumArgs ca, int nk1) {
-  __shared__ CumsumTile<kQ> tile;
-  if ((int)blockIdx.x >= nk1) {
-    chain_prep_body<T>(p, (int)blockIdx.x - nk1, threadIdx.x);
-    return;
-  }
-  cumsum_load<kQ, R, RAW>(ca, blockIdx.x, threadIdx.x, tile);
-  __syncthreads();
-  cumsum_scan<kQ>(ca, blockIdx.x, threadIdx.x / kWave, threadIdx.x % kWave, tile);
-}
-
-// Global -> LDS copies of 16 (4) bytes per lane from the wave-uniform base s
-// plus the lane's byte offset v: no vector address arithmetic per copy.  The
-// second form copies N blocks of 1 KB that lie 1 KB apart on both sides (the
-// instruction's offset applies to both addresses).  M0 holds the LDS
-// destination; nothing else in this kernel uses it.
-__device__ __forceinline__ void dma16_s(const void* s, uint32_t v, uint32_t lds_off) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :
-      : "v"(v), "s"(s), "s"(lds_off)
-      : "memory");
-}
-__device__ __forceinline__ void dma16x2_s(const void* s, uint32_t v, uint32_t lds_off) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1\n\t"
-      "global_load_lds_dwordx4 %0, %1 offset:1024"
-      :
-      : "v"(v), "s"(s), "s"(lds_off)
-      : "memory");
-}
-__device__ __forceinline__ void dma4_s(const void* s, uint32_t v, uint32_t lds_off) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dword %0, %1"
-      :
-      : "v"(v), "s"(s), "s"(lds_off)
-      : "memory");
-}
-__device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-template <typename U> __device__ __forceinline__ const U* uni(const U* q) {
-  const uint64_t v = (uint64_t)q;
-  return (const U*)(((uint64_t)uni((uint32_t)(v >> 32)) << 32) | uni((uint32_t)v));
-}
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ f32x16 mma32(bf16x8 a, bf16x8 b, f32x16 c) {
@@ -819,14 +708,6 @@ hipError_t launch_t(const ChainScanArgs& a, hipStream_t stream) {
   return a.wide ? launch_scan_t<T, 4, true, true>(a, stream) : launch_scan_t<T, 2, true, true>(a, stream);
 }
 
-template <typename T, typename R, bool RAW>
-hipError_t launch_prep_t(const ChainScanArgs& a, const CumsumArgs& ca, hipStream_t stream) {
-  const int64_t nk1 = cumsum_blocks(ca), nprep = (int64_t)a.batch * a.nsteps * a.ngroups;
-  if (nk1 + nprep > INT32_MAX) return hipErrorInvalidValue;
-  chain_prep_kernel<T, R, RAW><<<dim3((unsigned)(nk1 + nprep)), 256, 0, stream>>>(a, ca, (int)nk1);
-  return hipGetLastError();
-}
-
 }  // namespace
 
 size_t chain_scan_cb_bytes(int64_t steps) { return (size_t)steps * kTiles * 64 * sizeof(f32x4); }
@@ -886,9 +767,9 @@ ChainScanPlan chain_scan_plan(int64_t batch, int64_t steps, int64_t nheads, int6
 hipError_t launch_chain_prep(const ChainScanArgs& a, const CumsumArgs& ca, int dtype, hipStream_t stream) {
   if (ca.chunk != kQ || (ca.dt_raw && ca.raw_dtype != dtype)) return hipErrorInvalidValue;
   if (dtype == SSD_DTYPE_BF16)
-    return ca.dt_raw ? launch_prep_t<bf16, bf16, true>(a, ca, stream) : launch_prep_t<bf16, float, false>(a, ca, stream);
+    return ca.dt_raw ? launch_chain_prep_t<bf16, 4, bf16, true>(a, ca, stream) : launch_chain_prep_t<bf16, 4, float, false>(a, ca, stream);
   if (dtype == SSD_DTYPE_F16)
-    return ca.dt_raw ? launch_prep_t<f16, f16, true>(a, ca, stream) : launch_prep_t<f16, float, false>(a, ca, stream);
+    return ca.dt_raw ? launch_chain_prep_t<f16, 4, f16, true>(a, ca, stream) : launch_chain_prep_t<f16, 4, float, false>(a, ca, stream);
   return hipErrorInvalidValue;
 }
 

@@ -255,6 +255,12 @@ size_t chain_scan_cscale_bytes(int64_t steps);
 hipError_t launch_chain_prep(const ChainScanArgs& a, const CumsumArgs& ca, int dtype, hipStream_t stream);
 hipError_t launch_chain_scan(const ChainScanArgs& a, int dtype, hipStream_t stream);
 
+// The same walk for f32 inputs at d_state 64 / 128, never in segments
+// (ssd_chain_scan_f32.hip; no ct, cscale, seg_*, dskip, z)
+ChainScanPlan chain_scan_f32_plan(int64_t batch, int64_t steps, int64_t nheads, int64_t ngroups, int64_t dstate);
+hipError_t launch_chain_prep_f32(const ChainScanArgs& a, const CumsumArgs& ca, int dstate, hipStream_t stream);
+hipError_t launch_chain_scan_f32(const ChainScanArgs& a, int dstate, hipStream_t stream);
+
 // The whole forward in one launch for small states and short chains
 // (ssd_small.hip): d_state 16 / 32, chunk 64 / 128, at most kSmallMaxChunks
 // chunks per chain, f32 states kept in LDS; one workgroup per (b, h) chain.

@@ -311,7 +311,8 @@ def ssd_forward(X, A, B, C, chunk_size, dt=None, initial_states=None,
     * None (the default): the library's choice.  At d_state 128 with an even
       number of heads per group and enough work for the GPU the whole core
       runs as a walk along the (batch, head) chains with the state in float32
-      registers, and no states are handed over at all.  Otherwise f16 rows
+      registers, and no states are handed over at all (float32 inputs: at
+      d_state 64 / 128 with more than two chains per CU).  Otherwise f16 rows
       with a power-of-two scale per row ("f16s") wherever a 16-bit chunk_scan
       reads them: chunk 256 with d_state 64 / 128, and chunk 64 / 128 with
       chunk x d_state <= 8192.
