@@ -165,11 +165,17 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
 #pragma unroll
     for (int m = 2 * part; m < 2 * part + 2; ++m) dma16_s(xg + m * xst16, xv, xs_o + (uint32_t)((bf * 8 + 2 * m) * 1024));
   };
-  // C.B^T: this wave's five tiles go straight to registers
+  // C.B^T: this wave's five tiles go straight to registers, as buffer loads (as
+  // flat ones, which hold up the LDS counter, batch 4 x 4096 of 80 heads takes 172
+  // us instead of 168, 1 x 65536 710 instead of 690; with the gate and two heads per
+  // workgroup the buffer form spills)
   f32x4 cbv[5];
   auto load_cb = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) cbv[k] = *reinterpret_cast<const f32x4*>(cbg + (lane * 16 + k * 2048));
+    for (int k = 0; k < 5; ++k) {
+      if constexpr (EPI && HPW == 2) cbv[k] = *reinterpret_cast<const f32x4*>(cbg + (lane * 16 + k * 2048));
+      else cbv[k] = load16_b(cbg, lane * 16 + k * 2048);
+    }
   };
 
 #pragma unroll
