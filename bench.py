@@ -614,9 +614,11 @@ def main():
         fn()
         kernels[name] = kernel_entry(name, time_launches(fn, args.kernel_reps))
         pre_launches += 1 + args.kernel_reps
-    # the dominant kernel among those the forward runs: K2 + K3 as it runs them
+    # the dominant stage kernel: K2 + K3 as the stage path runs them
     # (chunk_state_passing), K4, K1 and K0 -- not the standalone chunk_state
-    # and state_passing rows, which stand in for it only as a breakdown
+    # and state_passing rows, which stand in for it only as a breakdown.  (Where
+    # ssd_forward runs the chain walk, whose launches have no entry point of
+    # their own, these rows describe the stage kernels beside it.)
     dom = max((k for k in kernels if k not in ("chunk_state", "state_passing")), key=lambda k: kernels[k]["ms"])
     kd = kernels[dom]
     if kd["bound"] == "hbm":

@@ -42,7 +42,7 @@
 // the exponentials) gains 2-4%, x's or y's traffic 12-18%.  Measured (us per
 // call, stage kernels -> walk): batch 8 x 2048 tokens, 128 heads, 8 groups, f16:
 // 368 -> 200, the layer span there 576 -> 382; batch 4 x 4096, 80 heads, bf16:
-// 208 -> 178 (3 segments); 1 x 65536, 80 heads: 828 -> 700 (12 segments).
+// 197 -> 168 (3 segments); 1 x 65536, 80 heads: 800 -> 694 (12 segments).
 // Slower: two 16-row halves per wave on 16x16x32 MFMAs (twice the LDS reads: 437
 // against 387 us for the layer span), the MFMAs of a step behind all its copies
 // (a copy stalls its wave while others queue: 6% of a step).
