@@ -12,12 +12,17 @@ tests/test_gpu_parity.py holds chunk_state).
 
 CPU: the per-lane LDS address formulas, restated and pinned to the source."""
 
+import os
+import re
+import subprocess
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import ssd_oracle as O
 from test_address_bounds import inside, pin
+from workloadsuite_amd import build
 from workloadsuite_amd import ssd as S
 
 DEV = "cuda"
@@ -126,6 +131,27 @@ def test_layer_span(dtype, b, L, h, g):
     torch.testing.assert_close(y.float(), ref.reshape(b, L, -1).float(), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", [(4, 512, 128, 8), (3, 1216, 96, 8), (1, 2752, 96, 16)])
+def test_layer_span_two_heads(dtype, b, L, h, g):
+    """The gated variant with two heads per workgroup: two whole-chain shapes, and
+    one whose groups of six heads are cut into segments.  Against the stage entry
+    points, 2e-2, and a second call gives the bits of the first."""
+    from test_layer_kernels import layer_case, split
+    print("CASE chain walk, layer span, two heads", dtype, b, L, h, g, flush=True)
+    proj, prm = layer_case(dtype, b=b, L=L, h=h, P=64, g=g, N=128)
+    x, z, B, C, dt = split(proj.to(DEV), h, 64, g, 128)
+    p = {k: v.to(DEV) for k, v in prm.items()}
+    y, y2 = (S.ssd_layer(x, z, B, C, dt, p["conv_w"], p["conv_b"], p["dt_bias"], p["A_log"], p["D"], 64, h) for _ in range(2))
+    X, dto, Acs, dec = S.layer_prep(x, dt, p["conv_w"], p["conv_b"], p["dt_bias"], p["A_log"], 64, h)
+    S_in, _ = S.chunk_state_passing(X, B, Acs, dec, dt=dto)
+    ref = S.chunk_scan(X, B, C, Acs, S_in, dt=dto, D=p["D"], z=z.reshape(b, L, h, 64))
+    torch.cuda.synchronize()
+    torch.testing.assert_close(y.float(), ref.reshape(b, L, -1).float(), rtol=2e-2, atol=2e-2)
+    assert torch.equal(y, y2)
+
+
 # ---------------------------------------------------------------------------
 # addresses (CPU)
 # ---------------------------------------------------------------------------
@@ -196,6 +222,44 @@ def test_lds_addresses():
             assert (img_c[slots][..., 0] == (32 * t + r)[:, None]).all()
             # S's lane values of K step kb: n = 16 kb + 8 hl + j
             assert (img_c[slots][..., 1] == (16 * kb + 8 * hl)[:, None] + np.arange(8)).all()
+
+
+@pytest.mark.parametrize("src", ["ssd_chain_scan.hip", "ssd_chain_scan_f32.hip"])
+def test_counted_waits(src, tmp_path):
+    """The compiled kernels: a barrier's counted wait leaves in flight only
+    accesses issued after the copies that the barrier publishes, and there are no
+    flat accesses, which may retire out of that order.  (The scan's first barrier
+    leaves the next step's x copies, its second none; the segment-state kernel's
+    leaves the copies of the step after next.)"""
+    out = tmp_path / "walk.s"
+    cmd = [build.hipcc(), *build.COMMON_FLAGS, *build.DEVICE_FLAGS, "-Wno-error", "--cuda-device-only", "-S",
+           os.path.join(build.CSRC, src), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True)
+    name, body, seen = None, [], 0
+    for ln in out.read_text().splitlines():
+        m = re.match(r"(_Z\w+):", ln)
+        if m:
+            name, body = m.group(1), []
+        elif name and re.match(r"\t[a-z]", ln):
+            body.append(ln.split(";")[0].strip())
+            if body[-1] != "s_endpgm" or "prep" in name:
+                continue
+            seen += 1
+            assert not [x for x in body if x.startswith("flat_")], name
+            waits = {}
+            for k, x in enumerate(body):
+                if x == "s_barrier":
+                    at, n = max((j, int(w.group(1))) for j in range(k) if (w := re.search(r"vmcnt\((\d+)\)", body[j])))
+                    ops = [y for y in body[:at] if re.match(r"(global|buffer)_", y)]
+                    waits[n] = len([y for y in ops[len(ops) - n:] if "_lds_" in y])
+            if "state_kernel" in name:
+                assert len(waits) == 1 and all(n == copies > 0 for n, copies in waits.items()), (name, waits)
+            elif "f32" in src:
+                assert waits == {0: 0, 40: 0}, (name, waits)
+            else:
+                gated = name.endswith("ELb1EEEvNS_13ChainScanArgsE")
+                assert waits == {0: 0, 9: 0, 8 if gated else 4: 4}, (name, waits)
+    assert seen == {"ssd_chain_scan.hip": 16, "ssd_chain_scan_f32.hip": 4}[src]
 
 
 def test_w_tiles():

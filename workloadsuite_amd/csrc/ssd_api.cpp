@@ -444,7 +444,7 @@ ssd::ChainScanPlan chain_plan(const ssd_dims* d, int dtype, const int64_t x_stri
   // lane offsets inside a step are 32-bit
   for (int64_t st : {x_strides[1], b_strides[1], c_strides[1], dt_strides ? dt_strides[1] : 0})
     if (st > (1 << 23)) return none;
-  if (f32 && y_strides[1] > (1 << 23)) return none;
+  if (y_strides[1] > (1 << 23) || (epi && epi->z_strides[1] > (1 << 23))) return none;
   const ssd::ChainScanPlan plan =
       f32 ? ssd::chain_scan_f32_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, d->dstate)
           : ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, epi != nullptr);

@@ -126,14 +126,16 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
   const uint32_t xs_o = uni(lds_offset(xs)) + (hh * 16 + w) * 1024;
   const uint32_t al_o = uni(lds_offset(al)) + hh * 256, dl_o = uni(lds_offset(dl)) + hh * 256;
   const uint32_t csl_o = uni(lds_offset(csl)) + hh * 256;
-  // lane offsets: blocks d = DPW wave + m of B and C, blocks w + 2 m of x
-  uint32_t bv[DPW], cv[DPW];
+  // lane offsets: blocks d = DPW wave + m of B and C, blocks w + 2 m of x (B's
+  // rows 8 further on lie in the same slots, so blocks m and m + 2 share one)
+  uint32_t bv[2], cv[DPW];
 #pragma unroll
   for (int m = 0; m < DPW; ++m) {
-    const int d = DPW * wave + m, row = 4 * d + crow;
-    bv[m] = (uint32_t)(row * (int)p.sbl + 8 * (cslot ^ bsw(row & 15))) * 2;
+    const int row = 4 * (DPW * wave + m) + crow;
+    if (m < 2) bv[m] = (uint32_t)(row * (int)p.sbl + 8 * (cslot ^ bsw(row & 15))) * 2;
     cv[m] = (uint32_t)(row * (kCT ? kN : (int)p.scl) + 8 * (cslot ^ (row & 15))) * 2;
   }
+  const int64_t bst8 = (int64_t)8 * p.sbl * 2;
   const uint32_t xv = (uint32_t)((8 * w + (lane >> 3)) * (int)p.sxl + 8 * ((lane & 7) ^ (lane >> 3))) * 2;
   const int64_t xst16 = (int64_t)16 * p.sxl * 2;
   const uint32_t dv = HAS_DT ? (uint32_t)(lane * (int)p.sdl) * 4 : 0;
@@ -159,23 +161,19 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
   auto issue_b = [&](int part) __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < DPW; ++m)
-      if ((2 * m) / DPW == part) dma16_s(bg, bv[m], bs_o + m * 1024);
+      if ((2 * m) / DPW == part) dma16_s(bg + (m >> 1) * bst8, bv[m & 1], bs_o + m * 1024);
   };
   auto issue_x = [&](int part, int bf) __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 2 * part; m < 2 * part + 2; ++m) dma16_s(xg + m * xst16, xv, xs_o + (uint32_t)((bf * 8 + 2 * m) * 1024));
   };
-  // C.B^T: this wave's five tiles go straight to registers, as buffer loads (as
-  // flat ones, which hold up the LDS counter, batch 4 x 4096 of 80 heads takes 172
-  // us instead of 168, 1 x 65536 710 instead of 690; with the gate and two heads per
-  // workgroup the buffer form spills)
+  // C.B^T: this wave's five tiles go straight to registers, as buffer loads.  Never
+  // as flat ones (what a load through a pointer that went through uni() becomes):
+  // those may retire ahead of older accesses, and vm_wait<NY> counts on the order.
   f32x4 cbv[5];
   auto load_cb = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      if constexpr (EPI && HPW == 2) cbv[k] = *reinterpret_cast<const f32x4*>(cbg + (lane * 16 + k * 2048));
-      else cbv[k] = load16_b(cbg, lane * 16 + k * 2048);
-    }
+    for (int k = 0; k < 5; ++k) cbv[k] = load16_b(cbg, lane * 16 + k * 2048);
   };
 
 #pragma unroll
@@ -230,10 +228,16 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
   const float dskip = EPI && p.dskip ? p.dskip[h] : 0.f;
   // y (and z): 16 rows of 64 bytes per instruction, 16-byte piece 2 (g & 1) + hl of the row in lane group g
   const int ypiece = 2 * (g & 1) + hl;
-  T* yg = reinterpret_cast<T*>(p.y) + (int64_t)b * p.syb + (int64_t)h * p.syh + (int64_t)i * p.syl + 32 * w + 8 * ypiece;
+  // (a wave-uniform base and the lane's 32-bit offset: one register less than a
+  // pointer per lane, and no vector arithmetic per step)
+  T* yg = reinterpret_cast<T*>(p.y) + (int64_t)b * p.syb + (int64_t)h * p.syh + 32 * w;
+  const uint32_t yv = (uint32_t)(i * (int)p.syl + 8 * ypiece) * 2;
   const T* zg = nullptr;
-  if constexpr (EPI)
-    zg = reinterpret_cast<const T*>(p.z) + (int64_t)b * p.szb + (int64_t)h * p.szh + (int64_t)i * p.szl + 32 * w + 8 * ypiece;
+  uint32_t zo = 0;
+  if constexpr (EPI) {
+    zg = reinterpret_cast<const T*>(p.z) + (int64_t)b * p.szb + (int64_t)h * p.szh + 32 * w;
+    zo = (uint32_t)(i * (int)p.szl + 8 * ypiece) * 2;
+  }
 
   // operand addresses (elements)
   const int q = i & 3, trow = 4 * hl + (i >> 2);  // transposing reads: rows 16 kb + trow (+ 8)
@@ -270,7 +274,9 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     __builtin_amdgcn_s_setprio(0);
     const float* ab = al[hh];
     const float a_own = ab[lane];
-    auto read_c = [&](f16x8 (&cf)[2], int kb) __attribute__((always_inline)) {
+    int co = coff;
+    if constexpr (EPI && HPW == 2) asm volatile("" : "+v"(co));  // (the eight addresses, kept over the steps, would not fit the registers)
+    auto read_c = [&, coff = co](f16x8 (&cf)[2], int kb) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) cf[t] = *reinterpret_cast<const f16x8*>(cl + (coff ^ (16 * kb)) + 32 * t * kN);
     };
@@ -344,7 +350,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int k = 0; k < 2; ++k) zv[EPI ? 2 * t + k : 0] = load8<T>(zg + ((int64_t)c * kQ + 32 * t + 16 * k) * p.szl);
+          for (int k = 0; k < 2; ++k) zv[EPI ? 2 * t + k : 0] = __builtin_bit_cast(frag8<T>, load16_g(zg + ((int64_t)c * kQ + 32 * t + 16 * k) * p.szl, zo));
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t) acc[t] = mma32(sf[kb], cf[kb & 1][t], acc[t]);
@@ -501,8 +507,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
         ob[j] = q2[1];
       }
       T* yr = yg + ((int64_t)c * kQ + 32 * t) * p.syl;
-      *reinterpret_cast<u32x4*>(yr) = oa;
-      *reinterpret_cast<u32x4*>(yr + 16 * p.syl) = ob;
+      store16_g(yr, yv, __builtin_bit_cast(f32x4, oa));
+      store16_g(yr + 16 * p.syl, yv, __builtin_bit_cast(f32x4, ob));
     }
     vm_wait<NY>();
     __syncthreads();

@@ -47,6 +47,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base) {
 __device__ __forceinline__ f32x4 load16_b(const void* base, uint32_t v) {
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc(base), v, 0, 0));
 }
+// The same as a global access (a generic pointer would make it a flat one, which
+// a counted wait on other accesses cannot hold apart from them).
+__device__ __forceinline__ f32x4 load16_g(const void* base, uint32_t v) {
+  typedef const f32x4 __attribute__((address_space(1))) * gptr;
+  return *(gptr)((const char __attribute__((address_space(1)))*)base + v);
+}
+__device__ __forceinline__ void store16_g(void* base, uint32_t v, f32x4 d) {
+  typedef f32x4 __attribute__((address_space(1))) * gptr;
+  *(gptr)((char __attribute__((address_space(1)))*)base + v) = d;
+}
 
 // The causal tiles (row tile t of l, column tile s of s, s <= t) in pairs 2 m +
 // w, one for each wave of a head: (t, s) = (kT[m] + kDT[m] w, kS[m] + kDS[m] w).
