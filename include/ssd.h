@@ -288,6 +288,19 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * actually run or time its kernels one by one. */
 int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype);
 
+/* How ssd_forward (gated 0) or ssd_layer_forward (gated 1; state_dtype
+ * SSD_DTYPE_F32) runs the core of d: as a chain walk, or segments 0 for the
+ * stage kernels.  For operands the walk takes as they are (16-byte aligned
+ * rows, no row stride above 2^23 elements), workspace of the size asked for.
+ * Host-only; without a device the answer is that for 256 CUs. */
+typedef struct ssd_walk_plan {
+  int64_t segments; /* of each (batch, head) chain; 0: not a walk */
+  int64_t steps;    /* 64-token steps per segment (the last may have fewer) */
+  int64_t heads;    /* per workgroup of the walk */
+  int64_t linked;   /* 1: a launch of its own forms the states entering the segments */
+} ssd_walk_plan;
+int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, ssd_walk_plan* plan);
+
 int ssd_forward(const ssd_dims* d, int dtype,
                 const void* x, const int64_t x_strides[4],
                 const float* a, const int64_t a_strides[3],

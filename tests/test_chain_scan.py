@@ -3,8 +3,8 @@ inputs at d_state 128 with at least ten (chain, 64-token step) pairs per CU.
 
 GPU: against the float64 oracle (chunked evaluation at 64), at shapes that
 take one segment, segments whose entering state each workgroup forms itself
-(up to 4) and segments that state_passing finishes, with ragged last
-segments, both types, dt, an initial state, strided operands and state rows
+(up to 4) and segments that state_passing finishes (each shape's plan is
+asserted), with ragged last segments, both types, dt, an initial state, strided operands and state rows
 outside f16's range.  y within 2e-2 (the 16-bit tolerance); the final state,
 whose products run on hi + lo pairs of the input type, to f32 accuracy: the
 pair is within 2^-17 of each product, so 3e-5 of max|state| (as
@@ -48,8 +48,8 @@ def check(Y, final, ref, fref, tol=2e-2):
 
 
 SHAPES = [
-    # b, L, h, g: one segment (512 chains of 6 steps); 2-4 segments; more than
-    # four (16 chains of 193 steps); a prime number of steps; six heads per group
+    # b, L, h, g: one segment (512 chains of 6 steps); eight; 49 (16 chains of
+    # 193 steps); a prime number of steps; six heads per group
     (8, 384, 64, 4),
     (2, 2496, 64, 8),
     (1, 12352, 16, 2),
@@ -58,11 +58,64 @@ SHAPES = [
 ]
 
 
+# b, L, h, g: segments, steps per segment, heads per workgroup, linked by a launch of their own
+PLANS = {
+    (8, 384, 64, 4): (1, 6, 2, False),
+    (2, 2496, 64, 8): (8, 5, 2, True),
+    (1, 12352, 16, 2): (49, 4, 2, True),
+    (1, 64 * 67, 48, 1): (17, 4, 2, True),
+    (3, 1088, 96, 16): (1, 17, 2, False),
+    # entering states formed by each workgroup: four segments (groups of 80 heads) and three (of six)
+    (3, 1216, 80, 1): (4, 5, 2, False),
+    (3, 1472, 48, 8): (3, 8, 2, False),
+    # groups of six heads, linked by a launch
+    (3, 2368, 24, 4): (7, 6, 2, True),
+    # strided operands
+    (2, 1344, 64, 4): (7, 3, 2, True),
+}
+GATED_PLANS = {
+    (8, 384, 128, 8): (1, 6, 4, False),
+    (2, 1216, 128, 8): (4, 5, 4, False),
+    (1, 2752, 64, 1): (15, 3, 4, True),
+    # two heads per workgroup
+    (4, 512, 128, 8): (1, 8, 2, False),
+    (3, 1216, 96, 8): (1, 19, 2, False),
+    (1, 2752, 96, 16): (5, 9, 2, True),
+    (3, 1472, 48, 8): (3, 8, 2, False),
+    (3, 1344, 96, 8): (3, 7, 2, False),
+}
+
+
+@pytest.mark.parametrize("gated", [False, True])
+def test_plans(gated):
+    """Every shape of the GPU tests below takes the walk it is there for (256 CUs)."""
+    for (b, L, h, g), want in (GATED_PLANS if gated else PLANS).items():
+        for dtype in (torch.bfloat16, torch.float16):
+            assert S.walk_plan(b, L, h, 64, 128, g, 64, dtype, gated=gated) == want, (b, L, h, g)
+    assert {k[:4] for k in SHAPES + MORE_SHAPES} <= set(PLANS)
+    assert {k for k in SPANS + SPANS_TWO} == set(GATED_PLANS)
+    # what the walk does not take: a named hand-over format, an odd number of heads per group, d_state 64, small calls
+    assert S.walk_plan(8, 384, 64, 64, 128, 4, 64, torch.float16, state_format="f16s") is None
+    assert S.walk_plan(8, 384, 64, 64, 128, 64, 64, torch.float16) is None
+    assert S.walk_plan(8, 384, 64, 64, 64, 4, 64, torch.float16) is None
+    assert S.walk_plan(1, 384, 64, 64, 128, 4, 64, torch.float16) is None
+
+
+def on_the_walk(b, L, h, g, dtype, gated=False):
+    """The call below runs the walk planned above also on this device."""
+    got = S.walk_plan(b, L, h, 64, 128, g, 64, dtype, gated=gated)
+    assert got == (GATED_PLANS if gated else PLANS)[b, L, h, g], got
+
+
+MORE_SHAPES = [(3, 1216, 80, 1), (3, 1472, 48, 8), (3, 2368, 24, 4)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,L,h,g", SHAPES)
+@pytest.mark.parametrize("b,L,h,g", SHAPES + MORE_SHAPES)
 @pytest.mark.parametrize("opts", [True, False])
 def test_forward(dtype, b, L, h, g, opts):
+    on_the_walk(b, L, h, g, dtype)
     print("CASE chain walk", dtype, b, L, h, g, opts, flush=True)
     X, A, B, C, dt, init = case(dtype, b, L, h, g, seed=L + h)
     dt, init = (dt, init) if opts else (None, None)
@@ -100,8 +153,10 @@ def test_state_rows_outside_f16():
 def test_strided_operands_match_contiguous_ones():
     """x, B, C as column slices of a wider tensor, A and dt transposed: the bits of the contiguous call."""
     print("CASE chain walk, strides", flush=True)
-    X, A, B, C, dt, init = (t.to(DEV) for t in case(torch.float16, 2, 1280, 64, 4, seed=9))
-    wide = torch.zeros(2, 1280, 64 * 64 + 2 * 4 * 128 + 16, device=DEV, dtype=torch.float16)
+    L = 1344
+    on_the_walk(2, L, 64, 4, torch.float16)
+    X, A, B, C, dt, init = (t.to(DEV) for t in case(torch.float16, 2, L, 64, 4, seed=9))
+    wide = torch.zeros(2, L, 64 * 64 + 2 * 4 * 128 + 16, device=DEV, dtype=torch.float16)
     xs, bs, cs = wide[..., 8:8 + 4096], wide[..., 4104:4104 + 512], wide[..., 4616:4616 + 512]
     xs.copy_(X.flatten(2)), bs.copy_(B.flatten(2)), cs.copy_(C.flatten(2))
     At, dtt = A.transpose(1, 2).contiguous().transpose(1, 2), dt.transpose(1, 2).contiguous().transpose(1, 2)
@@ -113,11 +168,51 @@ def test_strided_operands_match_contiguous_ones():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("what", ["x", "B", "C"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 64, 4), (3, 1216, 80, 1)])
+def test_one_bad_value(b, L, h, g, what, bad):
+    """An infinity or NaN reaches the outputs it belongs to (the products of a
+    32-token block see the whole block, as in the stage kernels) and no others:
+    those keep their bits."""
+    print("CASE chain walk, one bad value", b, L, h, g, what, bad, flush=True)
+    on_the_walk(b, L, h, g, torch.bfloat16)
+    X, A, B, C, dt, _ = (t.to(DEV) for t in case(torch.bfloat16, b, L, h, g, seed=1))
+    call = lambda: S.ssd_forward(X, A, B, C, 64, dt=dt, return_final_states=True)  # noqa: E731
+    Y0, f0 = call()
+    l, bb = 64 * (L // 128) + 37, b - 1  # noqa: E741
+    hit = torch.zeros_like(Y0, dtype=torch.bool)       # what may change
+    fhit = torch.zeros_like(f0, dtype=torch.bool)
+    if what == "x":
+        X[bb, l, 5, 9] = bad
+        hit[bb, l - l % 32:, 5, 9] = True
+        fhit[bb, 5, 9] = True
+    elif what == "B":
+        B[bb, l, 0, 77] = bad
+        hit[bb, l:, :h // g] = True
+        fhit[bb, :h // g, :, 77] = True
+    else:
+        C[bb, l, 0, 77] = bad
+        hit[bb, l, :h // g] = True
+    Y, final = call()
+    torch.cuda.synchronize()
+    assert torch.equal(Y[~hit], Y0[~hit]) and torch.equal(final[~fhit], f0[~fhit])
+    own = Y[bb, l, 5, 9] if what == "x" else Y[bb, l, :h // g]
+    assert not torch.isfinite(own).any()
+    if what != "C":
+        assert not torch.isfinite(final[fhit]).any()
+
+
+SPANS = [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,L,h,g", [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)])
+@pytest.mark.parametrize("b,L,h,g", SPANS)
 def test_layer_span(dtype, b, L, h, g):
-    """The gated variant (four heads per workgroup, two, and with segments)
-    against the stage entry points on the same prepared operands, 2e-2."""
+    """The gated variant with four heads per workgroup (one segment, four, and
+    fifteen) against the stage entry points on the same prepared operands, 2e-2."""
+    on_the_walk(b, L, h, g, dtype, gated=True)
     from test_layer_kernels import layer_case, split
     print("CASE chain walk, layer span", dtype, b, L, h, g, flush=True)
     proj, prm = layer_case(dtype, b=b, L=L, h=h, P=64, g=g, N=128)
@@ -131,13 +226,17 @@ def test_layer_span(dtype, b, L, h, g):
     torch.testing.assert_close(y.float(), ref.reshape(b, L, -1).float(), rtol=2e-2, atol=2e-2)
 
 
+SPANS_TWO = [(4, 512, 128, 8), (3, 1216, 96, 8), (1, 2752, 96, 16), (3, 1472, 48, 8), (3, 1344, 96, 8)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,L,h,g", [(4, 512, 128, 8), (3, 1216, 96, 8), (1, 2752, 96, 16)])
+@pytest.mark.parametrize("b,L,h,g", SPANS_TWO)
 def test_layer_span_two_heads(dtype, b, L, h, g):
-    """The gated variant with two heads per workgroup: two whole-chain shapes, and
-    one whose groups of six heads are cut into segments.  Against the stage entry
+    """The gated variant with two heads per workgroup: whole chains, and in
+    segments with groups of six and of twelve heads.  Against the stage entry
     points, 2e-2, and a second call gives the bits of the first."""
+    on_the_walk(b, L, h, g, dtype, gated=True)
     from test_layer_kernels import layer_case, split
     print("CASE chain walk, layer span, two heads", dtype, b, L, h, g, flush=True)
     proj, prm = layer_case(dtype, b=b, L=L, h=h, P=64, g=g, N=128)

@@ -41,11 +41,20 @@ def case(b, L, h, g, N, seed):
     return X, A, B, C, dt, init
 
 
+def test_plans():
+    """Every shape of the GPU tests takes the walk (256 CUs): whole chains, two heads per workgroup."""
+    for b, L, h, g, N, chunk in SHAPES + [(9, 256, 64, 8, 64, 64), (9, 256, 64, 8, 128, 64)]:
+        assert S.walk_plan(b, L, h, 64, N, g, chunk, torch.float32) == (1, L // 64, 2, False), (b, L, h, g, N)
+    assert S.walk_plan(8, 192, 64, 64, 64, 4, 64, torch.float32) is None   # one workgroup per CU
+    assert S.walk_plan(9, 192, 64, 64, 64, 64, 64, torch.float32) is None  # one head per group
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("b,L,h,g,N,chunk", SHAPES)
 @pytest.mark.parametrize("opts", [True, False])
 def test_forward(b, L, h, g, N, chunk, opts):
     print("CASE f32 chain walk", b, L, h, g, N, chunk, opts, flush=True)
+    assert S.walk_plan(b, L, h, 64, N, g, chunk, torch.float32) is not None
     X, A, B, C, dt, init = case(b, L, h, g, N, seed=L + h)
     dt, init = (dt, init) if opts else (None, None)
     hs = [0, 1, h // 2, h - 1]
@@ -65,6 +74,7 @@ def test_strided_operands_match_contiguous_ones(N):
     """x, B, C and dt as slices of wider tensors, A transposed: the bits of the contiguous call."""
     print("CASE f32 chain walk, strides", N, flush=True)
     b, L, h, g = 9, 256, 64, 8
+    assert S.walk_plan(b, L, h, 64, N, g, 64, torch.float32) is not None
     X, A, B, C, dt, init = (t.to(DEV) for t in case(b, L, h, g, N, seed=3))
     wide = torch.zeros(b, L, h * 64 + 2 * g * N + h + 12, device=DEV)
     at = [4, 4 + h * 64, 4 + h * 64 + g * N, 4 + h * 64 + 2 * g * N]

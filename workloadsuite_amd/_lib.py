@@ -35,6 +35,7 @@ EXPORTS = (
     "ssd_chunk_state_passing",
     "ssd_chunk_scan",
     "ssd_forward_chunk",
+    "ssd_forward_plan",
     "ssd_forward",
     "ssd_decode_step",
     "ssd_layer_prep",
@@ -47,6 +48,10 @@ EXPORTS = (
 class SSDDims(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int64) for n in
                 ("batch", "seqlen", "nheads", "headdim", "dstate", "ngroups", "chunk")]
+
+
+class SSDWalkPlan(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in ("segments", "steps", "heads", "linked")]
 
 
 class SSDEpilogue(ctypes.Structure):
@@ -80,6 +85,7 @@ _SIGNATURES = {
     "ssd_chunk_scan": (_int, [_dims_p, _int, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
                               _vp, _vp, _int, _vp, _vp, _i64p, _vp, _epi_p, _vp]),
     "ssd_forward_chunk": (ctypes.c_int64, [_dims_p, _int, _int]),
+    "ssd_forward_plan": (_int, [_dims_p, _int, _int, _int, ctypes.POINTER(SSDWalkPlan)]),
     "ssd_forward": (_int, [_dims_p, _int, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
                            _vp, _vp, _i64p, _vp, _vp, ctypes.c_size_t, _int, _vp]),
     "ssd_decode_step": (_int, [_dims_p, _int, _vp, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _vp, _i64p,

@@ -432,24 +432,29 @@ bool vec_rows(const void* p, const int64_t* strides, int n, int dtype) {
 
 // The plan of the core with f32 states as a chain walk (16-bit inputs at
 // d_state 128, f32 ones at 64 / 128), or nseg 0 where it does not apply or the
-// stage kernels are the faster way.
+// stage kernels are the faster way: for the shape, and for a call's operands.
+ssd::ChainScanPlan chain_shape_plan(const ssd_dims* d, int dtype, bool gated, size_t ws_bytes) {
+  const ssd::ChainScanPlan none{0, 0, false};
+  const bool f32 = dtype == SSD_DTYPE_F32;
+  if ((f32 && gated) || d->headdim != 64 || (f32 ? d->dstate != 64 && d->dstate != 128 : d->dstate != 128)) return none;
+  const ssd::ChainScanPlan plan =
+      f32 ? ssd::chain_scan_f32_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, d->dstate)
+          : ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, gated);
+  if (plan.nseg == 0 || chain_ws(d, dtype, plan.nseg).total > ws_bytes) return none;
+  return plan;
+}
+
 ssd::ChainScanPlan chain_plan(const ssd_dims* d, int dtype, const int64_t x_strides[4], const int64_t b_strides[4],
                               const int64_t c_strides[4], const int64_t* dt_strides, const void* y,
                               const int64_t y_strides[4], const ssd_epilogue* epi, size_t ws_bytes) {
   const ssd::ChainScanPlan none{0, 0, false};
-  const bool f32 = dtype == SSD_DTYPE_F32;
-  if ((f32 && epi) || d->headdim != 64 || (f32 ? d->dstate != 64 && d->dstate != 128 : d->dstate != 128)) return none;
   if (!vec_rows(y, y_strides, 4, dtype)) return none;
   if (epi && (!epi->z || !dt_strides || !vec_rows(epi->z, epi->z_strides, 4, dtype))) return none;
   // lane offsets inside a step are 32-bit
   for (int64_t st : {x_strides[1], b_strides[1], c_strides[1], dt_strides ? dt_strides[1] : 0})
     if (st > (1 << 23)) return none;
   if (y_strides[1] > (1 << 23) || (epi && epi->z_strides[1] > (1 << 23))) return none;
-  const ssd::ChainScanPlan plan =
-      f32 ? ssd::chain_scan_f32_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, d->dstate)
-          : ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, epi != nullptr);
-  if (plan.nseg == 0 || chain_ws(d, dtype, plan.nseg).total > ws_bytes) return none;
-  return plan;
+  return chain_shape_plan(d, dtype, epi != nullptr, ws_bytes);
 }
 
 int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan, CumsumArgs k1, const void* x, const int64_t x_strides[4],
@@ -709,6 +714,19 @@ size_t ssd_workspace_bytes(const ssd_dims* d, int state_dtype) {
 int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype) {
   if (check_dims_impl(d, dtype) != SSD_OK) return 0;
   return forward_dims(d, dtype, state_dtype).chunk;
+}
+
+int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, ssd_walk_plan* out) {
+  const int rc = check_dims_impl(d, dtype);
+  if (rc) return rc;
+  if (!out) return SSD_ERR_NULL_POINTER;
+  *out = ssd_walk_plan{0, 0, 0, 0};
+  if (state_dtype != SSD_DTYPE_F32) return SSD_OK;
+  const ssd_dims e = gated ? layer_core_dims(d, dtype) : forward_dims(d, dtype, state_dtype);
+  if (!gated && small_forward(&e, state_dtype)) return SSD_OK;
+  const ssd::ChainScanPlan plan = chain_shape_plan(&e, dtype, gated != 0, ws_layout(&e, state_dtype).total);
+  if (plan.nseg > 0) *out = ssd_walk_plan{plan.nseg, plan.seg_len, plan.wide ? 4 : 2, plan.nseg > ssd::kFoldSegs};
+  return SSD_OK;
 }
 
 int ssd_chunk_cumsum(const ssd_dims* d, const float* a, const int64_t a_strides[3],

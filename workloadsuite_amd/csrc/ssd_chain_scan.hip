@@ -56,10 +56,6 @@ namespace {
 constexpr int kQ = kStep;    // tokens per step
 constexpr int kP = 64;       // head dim
 constexpr int kN = 128;      // d_state
-// Up to this many segments, each workgroup of the scan forms its entering
-// state itself from the end states of the segments before it (as many reads as
-// state_passing's, no writes and one launch less); above, state_passing does.
-constexpr int kFoldSegs = 4;
 constexpr int kWBlocks = 6;  // 32 (s) x 16 (l) blocks of W
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));

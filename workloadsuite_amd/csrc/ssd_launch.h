@@ -241,6 +241,10 @@ struct ChainScanArgs {
   int batch, nsteps, nheads, ngroups, nseg, seg_len;
   bool wide = false;      // epilogue: four heads per workgroup instead of two
 };
+// Up to this many segments, each workgroup of the scan forms its entering
+// state itself from the end states of the segments before it (as many reads as
+// state_passing's, no writes and one launch less); above, state_passing does.
+constexpr int kFoldSegs = 4;
 // How the chains of a shape are cut: nseg segments of seg_len steps; nseg 0:
 // not supported, or the stage kernels are as fast.
 struct ChainScanPlan {

@@ -37,6 +37,7 @@ from . import _lib
 __all__ = [
     "ssd_forward",
     "forward_chunk",
+    "walk_plan",
     "ssd_forward_noalloc",
     "ssd_core",
     "chunk_cumsum",
@@ -247,6 +248,26 @@ def forward_chunk(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, d
     if q == 0:
         _lib.check(_lib.load().ssd_check_dims(ctypes.byref(d), _DTYPES[dtype]))
     return q
+
+
+class WalkPlan(NamedTuple):
+    """How a core runs as a walk along its (batch, head) chains (``walk_plan``)."""
+    segments: int  # of each chain
+    steps: int     # 64-token steps per segment
+    heads: int     # per workgroup
+    linked: bool   # the states entering the segments come from a launch of their own
+
+
+def walk_plan(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, dtype, state_dtype=torch.float32,
+              state_format=None, gated=False):
+    """How the library runs ``ssd_forward`` (``gated``: ``ssd_layer``) of these
+    dims, for operands it takes as they are: a WalkPlan, or None for the stage
+    kernels.  Without a device, as for 256 CUs."""
+    d = _lib.dims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size)
+    p = _lib.SSDWalkPlan()
+    _lib.check(_lib.load().ssd_forward_plan(ctypes.byref(d), _DTYPES[dtype], _handover(state_format, dtype, state_dtype),
+                                            int(gated), ctypes.byref(p)))
+    return WalkPlan(p.segments, p.steps, p.heads, bool(p.linked)) if p.segments else None
 
 
 # ssd_forward's per-call host work, kept per layout: the ctypes dims and
