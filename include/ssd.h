@@ -280,7 +280,8 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * SSD_STATE_F16S), L % 256 == 0 and dstate 64 / 128, a chunk of 64 or 128
  * runs at 256 unless that workspace would be larger than the caller's
  * chunk's (see ssd_forward_chunk).  Every chunking evaluates the same linear
- * recurrence (MR:152-161), so this changes rounding only. */
+ * recurrence (MR:152-161), so this changes rounding only.  final_states may be
+ * initial_states (the carried state updated in place). */
 /* The chunk length ssd_forward (and ssd_forward_noalloc) runs d's stage
  * kernels at, and sizes its workspace for, with this dtype and state_dtype:
  * d->chunk, or 256 where the rule above applies; 0 for invalid dims.  Host-only.  No counterpart in the reference (its
@@ -291,7 +292,8 @@ int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype);
 /* How ssd_forward (gated 0) or ssd_layer_forward (gated 1; state_dtype
  * SSD_DTYPE_F32) runs the core of d: as a chain walk, or segments 0 for the
  * stage kernels.  For operands the walk takes as they are (16-byte aligned
- * rows, no row stride above 2^23 elements), workspace of the size asked for.
+ * rows, no row stride above 2^23 elements), workspace of the size asked for;
+ * in_place: with final_states = initial_states.
  * Host-only; without a device the answer is that for 256 CUs. */
 typedef struct ssd_walk_plan {
   int64_t segments; /* of each (batch, head) chain; 0: not a walk */
@@ -299,7 +301,7 @@ typedef struct ssd_walk_plan {
   int64_t heads;    /* per workgroup of the walk */
   int64_t linked;   /* 1: a launch of its own forms the states entering the segments */
 } ssd_walk_plan;
-int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, ssd_walk_plan* plan);
+int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, int in_place, ssd_walk_plan* plan);
 
 int ssd_forward(const ssd_dims* d, int dtype,
                 const void* x, const int64_t x_strides[4],

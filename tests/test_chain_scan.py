@@ -12,6 +12,7 @@ tests/test_gpu_parity.py holds chunk_state).
 
 CPU: the per-lane LDS address formulas, restated and pinned to the source."""
 
+import ctypes
 import os
 import re
 import subprocess
@@ -22,7 +23,7 @@ import torch
 
 from oracle import ssd_oracle as O
 from test_address_bounds import inside, pin
-from workloadsuite_amd import build
+from workloadsuite_amd import _lib, build
 from workloadsuite_amd import ssd as S
 
 DEV = "cuda"
@@ -201,6 +202,38 @@ def test_one_bad_value(b, L, h, g, what, bad):
     assert not torch.isfinite(own).any()
     if what != "C":
         assert not torch.isfinite(final[fhit]).any()
+
+
+def test_in_place_state_waits_for_every_segment():
+    """With final_states = initial_states no workgroup of a cut chain may read the
+    initial state: at 6 x 16384 tokens of 112 heads 1008 workgroups share 512 places,
+    so the last segment of a chain can end before an earlier one starts."""
+    segs, steps, heads, linked = S.walk_plan(6, 16384, 112, 64, 128, 1, 64, torch.bfloat16)
+    assert (segs, linked) == (3, False) and 6 * segs * 112 // heads > 512
+    for b, L, h, g in [(6, 16384, 112, 1), (3, 1216, 80, 1), (3, 1472, 48, 8), (2, 2496, 64, 8)]:
+        assert S.walk_plan(b, L, h, 64, 128, g, 64, torch.bfloat16, in_place=True).linked
+    assert not S.walk_plan(8, 384, 64, 64, 128, 4, 64, torch.bfloat16, in_place=True).linked  # whole chains
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 64, 4), (3, 1216, 80, 1), (3, 1472, 48, 8), (2, 2496, 64, 8)])
+def test_state_updated_in_place(b, L, h, g):
+    """ssd_forward of the C ABI with final_states = initial_states: y and the state
+    of a call with two buffers (to the order in which the segments are linked)."""
+    print("CASE chain walk, in place", b, L, h, g, flush=True)
+    X, A, B, C, dt, init = (t.to(DEV) for t in case(torch.float16, b, L, h, g, seed=2))
+    Y0, f0 = S.ssd_forward(X, A, B, C, 64, dt=dt, initial_states=init, return_final_states=True)
+    n = S.workspace_bytes(b, L, h, 64, 128, g, 64)
+    ws, Y = torch.empty(n, dtype=torch.uint8, device=DEV), torch.empty_like(X)
+    d, lib = _lib.dims(b, L, h, 64, 128, g, 64), _lib.load()
+    st = _lib.strides
+    _lib.check(lib.ssd_forward(ctypes.byref(d), _lib.DTYPE_F16, X.data_ptr(), st(X), A.data_ptr(), st(A), B.data_ptr(), st(B),
+                               C.data_ptr(), st(C), dt.data_ptr(), st(dt), init.data_ptr(), Y.data_ptr(), st(Y),
+                               init.data_ptr(), ws.data_ptr(), n, _lib.DTYPE_F32, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    # one f32 rounding per linked segment apart; y one f16 rounding where that crosses a boundary
+    torch.testing.assert_close(init, f0, rtol=0, atol=1e-6 * f0.abs().max().item())
+    torch.testing.assert_close(Y.float(), Y0.float(), rtol=2e-3, atol=2e-3)
 
 
 SPANS = [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)]

@@ -85,7 +85,7 @@ _SIGNATURES = {
     "ssd_chunk_scan": (_int, [_dims_p, _int, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
                               _vp, _vp, _int, _vp, _vp, _i64p, _vp, _epi_p, _vp]),
     "ssd_forward_chunk": (ctypes.c_int64, [_dims_p, _int, _int]),
-    "ssd_forward_plan": (_int, [_dims_p, _int, _int, _int, ctypes.POINTER(SSDWalkPlan)]),
+    "ssd_forward_plan": (_int, [_dims_p, _int, _int, _int, _int, ctypes.POINTER(SSDWalkPlan)]),
     "ssd_forward": (_int, [_dims_p, _int, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
                            _vp, _vp, _i64p, _vp, _vp, ctypes.c_size_t, _int, _vp]),
     "ssd_decode_step": (_int, [_dims_p, _int, _vp, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _vp, _i64p,

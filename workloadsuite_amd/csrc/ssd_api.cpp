@@ -426,6 +426,13 @@ ChainWs chain_ws(const ssd_dims* d, int dtype, int nseg) {
   return w;
 }
 
+// The final states overlap the initial ones (both [b, h, P, N] f32).
+bool in_place(const ssd_dims* d, const float* init, const float* final_states) {
+  const uintptr_t i = reinterpret_cast<uintptr_t>(init), f = reinterpret_cast<uintptr_t>(final_states);
+  const uintptr_t n = (uintptr_t)(d->batch * d->nheads * d->headdim * d->dstate) * sizeof(float);
+  return init && final_states && i < f + n && f < i + n;
+}
+
 bool vec_rows(const void* p, const int64_t* strides, int n, int dtype) {
   return check_vec_operand(p, strides, n, dtype) == SSD_OK;
 }
@@ -509,6 +516,7 @@ int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan,
   p.nseg = plan.nseg;
   p.seg_len = plan.seg_len;
   p.wide = plan.wide;
+  p.linked = ssd::chain_scan_linked(plan.nseg, in_place(d, initial_states, final_states));
   const int n = (int)d->dstate;
   const bool f32 = dtype == SSD_DTYPE_F32;
   int rc;
@@ -716,7 +724,7 @@ int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype) {
   return forward_dims(d, dtype, state_dtype).chunk;
 }
 
-int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, ssd_walk_plan* out) {
+int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, int in_place, ssd_walk_plan* out) {
   const int rc = check_dims_impl(d, dtype);
   if (rc) return rc;
   if (!out) return SSD_ERR_NULL_POINTER;
@@ -725,7 +733,7 @@ int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, s
   const ssd_dims e = gated ? layer_core_dims(d, dtype) : forward_dims(d, dtype, state_dtype);
   if (!gated && small_forward(&e, state_dtype)) return SSD_OK;
   const ssd::ChainScanPlan plan = chain_shape_plan(&e, dtype, gated != 0, ws_layout(&e, state_dtype).total);
-  if (plan.nseg > 0) *out = ssd_walk_plan{plan.nseg, plan.seg_len, plan.wide ? 4 : 2, plan.nseg > ssd::kFoldSegs};
+  if (plan.nseg > 0) *out = ssd_walk_plan{plan.nseg, plan.seg_len, plan.wide ? 4 : 2, ssd::chain_scan_linked(plan.nseg, in_place != 0)};
   return SSD_OK;
 }
 

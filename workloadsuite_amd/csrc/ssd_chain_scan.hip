@@ -198,7 +198,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
 #pragma unroll
       for (int j = 0; j < 16; ++j) st[nt][j] = 0.f;
     const int64_t bh = (int64_t)b * p.nheads + h;
-    if (p.nseg > kFoldSegs) {
+    if (p.linked) {
       load_s(p.seg_states + (((int64_t)b * p.nseg + seg) * p.nheads + h) * (kP * kN), st);
     } else {
       // the state entering the segment, from the end states of those before it
@@ -680,7 +680,7 @@ hipError_t launch_state_t(const ChainScanArgs& a, hipStream_t stream) {
   auto kern = a.dt ? chain_state_kernel<T, HPW, true> : chain_state_kernel<T, HPW, false>;
   kern<<<dim3((unsigned)grid), dim3(128 * HPW), 0, stream>>>(a);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.nseg <= kFoldSegs) return e;
+  if (e != hipSuccess || !a.linked) return e;
   // the state entering each segment
   StatePassingArgs sp;
   sp.states = a.seg_states;

@@ -240,11 +240,15 @@ struct ChainScanArgs {
   int64_t szb = 0, szl = 0, szh = 0;
   int batch, nsteps, nheads, ngroups, nseg, seg_len;
   bool wide = false;      // epilogue: four heads per workgroup instead of two
+  bool linked = false;    // state_passing forms the states entering the segments (chain_scan_linked)
 };
 // Up to this many segments, each workgroup of the scan forms its entering
-// state itself from the end states of the segments before it (as many reads as
-// state_passing's, no writes and one launch less); above, state_passing does.
+// state itself from the initial state and the end states of the segments before
+// it (as many reads as state_passing's, no writes and one launch less); above,
+// state_passing does.  It also does where the final state overwrites the initial
+// one: a chain's last segment may be done before another of its segments starts.
 constexpr int kFoldSegs = 4;
+inline bool chain_scan_linked(int nseg, bool in_place) { return nseg > kFoldSegs || (nseg > 1 && in_place); }
 // How the chains of a shape are cut: nseg segments of seg_len steps; nseg 0:
 // not supported, or the stage kernels are as fast.
 struct ChainScanPlan {

@@ -259,14 +259,15 @@ class WalkPlan(NamedTuple):
 
 
 def walk_plan(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, dtype, state_dtype=torch.float32,
-              state_format=None, gated=False):
+              state_format=None, gated=False, in_place=False):
     """How the library runs ``ssd_forward`` (``gated``: ``ssd_layer``) of these
-    dims, for operands it takes as they are: a WalkPlan, or None for the stage
+    dims, for operands it takes as they are (``in_place``: with the final state
+    written over the initial one, as the C ABI allows): a WalkPlan, or None for the stage
     kernels.  Without a device, as for 256 CUs."""
     d = _lib.dims(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size)
     p = _lib.SSDWalkPlan()
     _lib.check(_lib.load().ssd_forward_plan(ctypes.byref(d), _DTYPES[dtype], _handover(state_format, dtype, state_dtype),
-                                            int(gated), ctypes.byref(p)))
+                                            int(gated), int(in_place), ctypes.byref(p)))
     return WalkPlan(p.segments, p.steps, p.heads, bool(p.linked)) if p.segments else None
 
 
