@@ -151,6 +151,44 @@ def test_state_rows_outside_f16():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 64, 4), (3, 1216, 80, 1), (2, 2496, 64, 8)])
+@pytest.mark.parametrize("small", [-12, -20, -24])
+def test_small_entries_of_a_state_row(dtype, b, L, h, g, small):
+    """C picks entries 2^small below their row's largest: with the row scaled to
+    [2^14, 2^15) they keep f16's 11 bits down to 2^-29 of it, so y is within the
+    rounding of S (half an ulp of 11 bits: 2^-11) and its own (2^-11 in f16, 2^-8
+    in bf16)."""
+    print("CASE chain walk, small entries", dtype, b, L, h, g, small, flush=True)
+    on_the_walk(b, L, h, g, dtype)
+    gen = torch.Generator().manual_seed(4)
+    init = torch.zeros(b, h, 64, 128)
+    init[..., 3] = 1 + torch.rand(b, h, 64, generator=gen)             # the row's largest
+    init[..., 40] = (1 + torch.rand(b, h, 64, generator=gen)) * 2.0 ** small
+    C = torch.zeros(b, L, g, 128)
+    C[..., 40] = 2.0 ** min(-small, 15)
+    X, A, B = torch.zeros(b, L, h, 64), torch.zeros(b, L, h), torch.zeros(b, L, g, 128)
+    Y = S.ssd_forward(X.to(DEV, dtype), A.to(DEV), B.to(DEV, dtype), C.to(DEV, dtype), 64, initial_states=init.to(DEV))
+    want = (init[..., 40].double() * 2.0 ** min(-small, 15)).to(DEV)[:, None]
+    eps = 2.0 ** -11 + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+    assert ((Y.double() - want).abs() <= 1.01 * eps * want).all()
+
+
+@pytest.mark.gpu
+def test_scales_of_c_and_s_cancel():
+    """C near bf16's largest values times a tiny state: the two scales are
+    multiplied first, so that neither alone overflows the sum."""
+    print("CASE chain walk, scales cancel", flush=True)
+    b, L, h, g = 8, 384, 64, 4
+    on_the_walk(b, L, h, g, torch.bfloat16)
+    init = torch.full((b, h, 64, 128), 2.0 ** -80, device=DEV)
+    C = torch.full((b, L, g, 128), 2.0 ** 114, device=DEV, dtype=torch.bfloat16)
+    X, A = torch.zeros(b, L, h, 64, device=DEV, dtype=torch.bfloat16), torch.zeros(b, L, h, device=DEV)
+    Y = S.ssd_forward(X, A, torch.zeros_like(C), C, 64, initial_states=init)
+    assert (Y == 2.0 ** 41).all()
+
+
+@pytest.mark.gpu
 def test_strided_operands_match_contiguous_ones():
     """x, B, C as column slices of a wider tensor, A and dt transposed: the bits of the contiguous call."""
     print("CASE chain walk, strides", flush=True)

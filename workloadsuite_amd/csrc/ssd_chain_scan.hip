@@ -21,10 +21,8 @@
 //   * S^T tiles (rows n, columns p) are accumulators; the n rows of a tile are
 //     dealt out (by the addresses of the transposing B reads) so that a lane's
 //     values are 8 consecutive n, the A operand of the off-diagonal product.
-//     They are rounded to f16 there, as SSD_STATE_F16S rounds states, with a
-//     power-of-two scale per row p where a row's largest magnitude lies outside
-//     [2^-9, 2^15) (inside, f16 holds the row as it is: what the scale could
-//     still save is below 2^-16 of the row's maximum).
+//     They are rounded to f16 there, as SSD_STATE_F16S rounds states: with a
+//     power-of-two scale per row p, the row's largest magnitude in [2^14, 2^15).
 //   * y^T tiles (rows p, columns l) start as the off-diagonal product, are
 //     scaled by exp(Acs[l]), and take the diagonal product on top.
 //   * W = decay . C.B^T is formed once per head, its ten causal 16 x 16 tiles
@@ -271,7 +269,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     const float* ab = al[hh];
     const float a_own = ab[lane];
     int co = coff;
-    if constexpr (EPI && HPW == 2) asm volatile("" : "+v"(co));  // (the eight addresses, kept over the steps, would not fit the registers)
+    if constexpr (EPI) asm volatile("" : "+v"(co));  // (the eight addresses, kept over the steps, would not fit the registers)
     auto read_c = [&, coff = co](f16x8 (&cf)[2], int kb) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) cf[t] = *reinterpret_cast<const f16x8*>(cl + (coff ^ (16 * kb)) + 32 * t * kN);
@@ -315,25 +313,21 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
-    // rows outside f16's comfortable range take a power-of-two scale each
-    const bool plain = __builtin_amdgcn_ballot_w64(!(m == 0.f || (m >= 0x1p-9f && m < 0x1p15f))) == 0;
-    f16x8 sf[8];
-    auto f16_rows = [&](auto SCALED, float sc) __attribute__((always_inline)) {
+    const int e = m > 0.f ? min(max(__builtin_amdgcn_frexp_expf(m) - 15, -100), 100) : 0;
+    const float sc = __builtin_ldexpf(1.f, -e);
+    if (hl == 0) rsl[wave][r] = __builtin_ldexpf(1.f, e);
+    // (scaled and rounded by one v_fma_mixlo / mixhi per value: the opaque -0
+    // addend keeps the compiler from making it a product and a conversion)
+    float nz = -0.f;
+    asm("" : "+v"(nz));
+    auto f16_rows = [&](int kb) __attribute__((always_inline)) {
+      f16x8 v;
 #pragma unroll
-      for (int kb = 0; kb < 8; ++kb) {
-        f32x8 v;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = decltype(SCALED)::value ? st[kb >> 1][8 * (kb & 1) + j] * sc : st[kb >> 1][8 * (kb & 1) + j];
-        sf[kb] = __builtin_convertvector(v, f16x8);
-      }
+      for (int j = 0; j < 8; ++j) v[j] = (f16)__builtin_fmaf(st[kb >> 1][8 * (kb & 1) + j], sc, nz);
+      return v;
     };
-    if (plain) {
-      f16_rows(std::false_type(), 1.f);
-    } else {
-      const int e = m > 0.f ? min(max(__builtin_amdgcn_frexp_expf(m) - 15, -100), 100) : 0;
-      if (hl == 0) rsl[wave][r] = __builtin_ldexpf(1.f, e);
-      f16_rows(std::true_type(), __builtin_ldexpf(1.f, -e));
-    }
+    f16x8 sf[2];
+    sf[0] = f16_rows(0);
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) {
       if (kb < 7) read_c(cf[(kb + 1) & 1], kb + 1);
@@ -349,7 +343,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
           for (int k = 0; k < 2; ++k) zv[EPI ? 2 * t + k : 0] = __builtin_bit_cast(frag8<T>, load16_g(zg + ((int64_t)c * kQ + 32 * t + 16 * k) * p.szl, zo));
       }
 #pragma unroll
-      for (int t = 0; t < 2; ++t) acc[t] = mma32(sf[kb], cf[kb & 1][t], acc[t]);
+      for (int t = 0; t < 2; ++t) acc[t] = mma32(sf[kb & 1], cf[kb & 1][t], acc[t]);
+      if (kb < 7) sf[(kb + 1) & 1] = f16_rows(kb + 1);
       // the state's decay, its value entering the step being taken
 #pragma unroll
       for (int j = 0; j < 8; ++j) st[kb >> 1][8 * (kb & 1) + j] *= dec;
@@ -369,22 +364,20 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
         store4<T>(&wl[hh][woff[kDI[kb]] + ((t0 >> 1) * 2 + s0) * 512 + (t0 & 1) * 128], __builtin_convertvector(v, vec4<T>));
       }
     }
+    // rows p carry their scale, columns l exp(Acs[l]) and C's scale
+    float ev[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      float ev = __builtin_amdgcn_exp2f(el[t] * kLog2e);
-      if constexpr (kCT) ev *= csl[hh][32 * t + r];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) acc[t][j] *= ev;
+      ev[t] = __builtin_amdgcn_exp2f(el[t] * kLog2e);
+      if constexpr (kCT) ev[t] *= csl[hh][32 * t + r];
     }
-    if (!plain) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const f32x4 rs = *reinterpret_cast<const f32x4*>(&rsl[wave][8 * k + 4 * hl]);
+    for (int k = 0; k < 4; ++k) {
+      const f32x4 rs = *reinterpret_cast<const f32x4*>(&rsl[wave][8 * k + 4 * hl]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int jj = 0; jj < 4; ++jj) acc[t][4 * k + jj] *= rs[jj];
-      }
+        for (int jj = 0; jj < 4; ++jj) acc[t][4 * k + jj] *= rs[jj] * ev[t];
     }
     if (c < last) bg += bst;
     if (c + 1 < last) xg += xst;
