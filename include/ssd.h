@@ -300,6 +300,7 @@ typedef struct ssd_walk_plan {
   int64_t steps;    /* 64-token steps per segment (the last may have fewer) */
   int64_t heads;    /* per workgroup of the walk */
   int64_t linked;   /* 1: a launch of its own forms the states entering the segments */
+  int64_t hilo;     /* 1: the state enters C.S as a hi + lo pair of the input type; 0: as f16 rows with a scale each (f32 inputs: as it is) */
 } ssd_walk_plan;
 int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, int in_place, ssd_walk_plan* plan);
 

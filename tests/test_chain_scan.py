@@ -59,31 +59,34 @@ SHAPES = [
 ]
 
 
-# b, L, h, g: segments, steps per segment, heads per workgroup, linked by a launch of their own
+# b, L, h, g: segments, steps per segment, heads per workgroup, linked by a launch of their own, S as a hi + lo pair
 PLANS = {
-    (8, 384, 64, 4): (1, 6, 2, False),
-    (2, 2496, 64, 8): (8, 5, 2, True),
-    (1, 12352, 16, 2): (49, 4, 2, True),
-    (1, 64 * 67, 48, 1): (17, 4, 2, True),
-    (3, 1088, 96, 16): (1, 17, 2, False),
+    (8, 384, 64, 4): (1, 6, 2, False, False),
+    (2, 2496, 64, 8): (8, 5, 2, True, False),
+    (1, 12352, 16, 2): (49, 4, 2, True, False),
+    (1, 64 * 67, 48, 1): (17, 4, 2, True, False),
+    (3, 1088, 96, 16): (1, 17, 2, False, False),
     # entering states formed by each workgroup: four segments (groups of 80 heads) and three (of six)
-    (3, 1216, 80, 1): (4, 5, 2, False),
-    (3, 1472, 48, 8): (3, 8, 2, False),
+    (3, 1216, 80, 1): (4, 5, 2, False, False),
+    (3, 1472, 48, 8): (3, 8, 2, False, False),
     # groups of six heads, linked by a launch
-    (3, 2368, 24, 4): (7, 6, 2, True),
+    (3, 2368, 24, 4): (7, 6, 2, True, False),
     # strided operands
-    (2, 1344, 64, 4): (7, 3, 2, True),
+    (2, 1344, 64, 4): (7, 3, 2, True, False),
 }
 GATED_PLANS = {
-    (8, 384, 128, 8): (1, 6, 4, False),
-    (2, 1216, 128, 8): (4, 5, 4, False),
-    (1, 2752, 64, 1): (15, 3, 4, True),
+    (8, 384, 128, 8): (1, 6, 4, False, True),
+    (2, 1216, 128, 8): (4, 5, 4, False, True),
+    (1, 2752, 64, 1): (15, 3, 4, True, True),
     # two heads per workgroup
-    (4, 512, 128, 8): (1, 8, 2, False),
-    (3, 1216, 96, 8): (1, 19, 2, False),
-    (1, 2752, 96, 16): (5, 9, 2, True),
-    (3, 1472, 48, 8): (3, 8, 2, False),
-    (3, 1344, 96, 8): (3, 7, 2, False),
+    (4, 512, 128, 8): (1, 8, 2, False, False),
+    (3, 1216, 96, 8): (1, 19, 2, False, True),
+    (1, 2752, 96, 16): (5, 9, 2, True, True),
+    (3, 1472, 48, 8): (3, 8, 2, False, True),
+    (3, 1344, 96, 8): (3, 7, 2, False, True),
+    # lengths that 256 divides: four heads per workgroup, two (one segment above), and two segments of groups of six
+    (8, 256, 128, 8): (1, 4, 4, False, False),
+    (5, 1024, 48, 8): (2, 8, 2, False, False),
 }
 
 
@@ -246,7 +249,7 @@ def test_in_place_state_waits_for_every_segment():
     """With final_states = initial_states no workgroup of a cut chain may read the
     initial state: at 6 x 16384 tokens of 112 heads 1008 workgroups share 512 places,
     so the last segment of a chain can end before an earlier one starts."""
-    segs, steps, heads, linked = S.walk_plan(6, 16384, 112, 64, 128, 1, 64, torch.bfloat16)
+    segs, _, heads, linked, _ = S.walk_plan(6, 16384, 112, 64, 128, 1, 64, torch.bfloat16)
     assert (segs, linked) == (3, False) and 6 * segs * 112 // heads > 512
     for b, L, h, g in [(6, 16384, 112, 1), (3, 1216, 80, 1), (3, 1472, 48, 8), (2, 2496, 64, 8)]:
         assert S.walk_plan(b, L, h, 64, 128, g, 64, torch.bfloat16, in_place=True).linked
@@ -274,7 +277,85 @@ def test_state_updated_in_place(b, L, h, g):
     torch.testing.assert_close(Y.float(), Y0.float(), rtol=2e-3, atol=2e-3)
 
 
-SPANS = [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)]
+SPANS = [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1), (8, 256, 128, 8)]
+
+
+# chunk 128, odd multiples: one segment, four, fourteen linked ones, three of groups of six heads
+CHUNK_128 = {(4, 640, 64, 8): (1, 10, 2, False, True), (3, 1152, 80, 1): (4, 5, 2, False, True),
+             (1, 2688, 64, 8): (14, 3, 2, True, True), (3, 1152, 48, 8): (3, 6, 2, False, True)}
+
+
+def test_state_operand_follows_the_stage_kernels():
+    """S enters C.S as a hi + lo pair where the stage kernels take it so (chunk
+    128, the gate at lengths that 256 does not divide), else as f16 rows."""
+    for dtype in (torch.bfloat16, torch.float16):
+        for (b, L, h, g), want in CHUNK_128.items():
+            assert S.walk_plan(b, L, h, 64, 128, g, 128, dtype) == want
+        for b, L, h, g, chunk, gated, hilo in [(4, 640, 64, 8, 64, False, False), (4, 1024, 80, 1, 128, False, False),
+                                               (4, 1024, 80, 1, 256, False, False), (8, 384, 128, 8, 128, True, True),
+                                               (8, 512, 128, 8, 128, True, False), (8, 512, 128, 8, 64, True, False)]:
+            assert S.walk_plan(b, L, h, 64, 128, g, chunk, dtype, gated=gated).hilo == hilo, (L, chunk, gated)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", list(CHUNK_128))
+@pytest.mark.parametrize("opts", [True, False])
+def test_forward_chunk_128(dtype, b, L, h, g, opts):
+    """As test_forward, at chunk 128; then a state whose entries nearly cancel:
+    y = S[3] - S[40] with S[3] = (1 + 1.5 2^-11) S[40], which 11 bits of S do not
+    resolve.  A bf16 pair of values below 2 is within 2^-17 of each (2^-16 of the
+    larger binade), an f16 pair closer; y's own rounding is 2^-8 (bf16)."""
+    print("CASE chain walk, chunk 128", dtype, b, L, h, g, opts, flush=True)
+    assert S.walk_plan(b, L, h, 64, 128, g, 128, dtype) == CHUNK_128[b, L, h, g]
+    X, A, B, C, dt, init = case(dtype, b, L, h, g, seed=L + h)
+    dt, init = (dt, init) if opts else (None, None)
+    hs = [0, 1, h // 2, h - 1]
+    grp = [k // (h // g) for k in hs]
+    ref, fref = O.ssd_chunked(X[:, :, hs], A[:, :, hs], B[:, :, grp], C[:, :, grp], 64,
+                              dt=None if dt is None else dt[:, :, hs], initial_states=None if init is None else init[:, hs])
+    d = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    Y, final = S.ssd_forward(d(X), d(A), d(B), d(C), 128, dt=d(dt), initial_states=d(init), return_final_states=True)
+    check(Y[:, :, hs], final[:, hs], ref, fref)
+    state = torch.zeros(b, h, 64, 128, device=DEV)
+    state[..., 40] = 1 + torch.rand(b, h, 64, device=DEV)
+    state[..., 3] = state[..., 40] * (1 + 1.5 * 2.0 ** -11)
+    C = torch.zeros(b, L, g, 128, device=DEV, dtype=dtype)
+    C[..., 3], C[..., 40] = 1, -1
+    zero = lambda t: torch.zeros_like(t, device=DEV)  # noqa: E731
+    Y = S.ssd_forward(zero(X), zero(A), zero(B), C, 128, dt=d(dt), initial_states=state)
+    want = (state[..., 3].double() - state[..., 40].double())[:, None]
+    assert ((Y.double() - want).abs() <= 2 * 2.0 ** -16 + 2.0 ** -8 * want).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 128, 8), (2, 1216, 128, 8), (3, 1216, 96, 8), (3, 1472, 48, 8)])
+def test_layer_span_resolves_the_state(dtype, b, L, h, g):
+    """The same near-cancellation in the gated walk: S[3] - S[40] = 1.5 2^-11 S[40]
+    from the first two tokens, read by all from the second 64 on."""
+    print("CASE chain walk, gated, near-cancelling state", dtype, b, L, h, g, flush=True)
+    on_the_walk(b, L, h, g, dtype, gated=True)
+    assert GATED_PLANS[b, L, h, g][4]
+    x = torch.zeros(b, L, h * 64, device=DEV)
+    x[:, 0] = x[:, 1] = 1 + torch.rand(b, h * 64, device=DEV)
+    B, C = torch.zeros(2, b, L, g, 128, device=DEV, dtype=dtype)
+    B[:, 0, :, 3] = B[:, 0, :, 40] = 1
+    B[:, 1, :, 3] = 1.5 * 2.0 ** -11
+    C[..., 3], C[..., 40] = 1, -1
+    z = torch.full((b, L, h * 64), 8.0, device=DEV, dtype=dtype)
+    dt = torch.full((b, L, h), 0.5, device=DEV, dtype=dtype)
+    w = torch.zeros(h * 64, 1, 4, device=DEV, dtype=dtype)
+    w[..., 3] = 1
+    zero = torch.zeros(h, device=DEV)
+    x = x.to(dtype)
+    y = S.ssd_layer(x, z, B, C, dt, w, None, zero.to(dtype), zero - 30, zero, 64, h)
+    # x as the conv leaves it, dt = softplus(0.5), decays 1 - 1e-10
+    xv = torch.nn.functional.silu(x[:, 0].double()).to(dtype).double() * torch.nn.functional.softplus(dt[0, 0, 0].double())
+    gate = torch.nn.functional.silu(torch.tensor(8.0, dtype=torch.float64, device=DEV))
+    want = (xv * 1.5 * 2.0 ** -11 * gate)[:, None]
+    # S below 4: a pair is within 2^-15 of each entry; x's rounding after the conv may differ by an ulp (2^-8)
+    assert ((y[:, 64:].double() - want).abs() <= gate * 2 * 2.0 ** -15 + 2 * 2.0 ** -8 * want).all()
 
 
 @pytest.mark.gpu
@@ -282,7 +363,7 @@ SPANS = [(8, 384, 128, 8), (2, 1216, 128, 8), (1, 2752, 64, 1)]
 @pytest.mark.parametrize("b,L,h,g", SPANS)
 def test_layer_span(dtype, b, L, h, g):
     """The gated variant with four heads per workgroup (one segment, four, and
-    fifteen) against the stage entry points on the same prepared operands, 2e-2."""
+    fifteen; S as a hi + lo pair, and at 256 tokens as f16 rows) against the stage entry points on the same prepared operands, 2e-2."""
     on_the_walk(b, L, h, g, dtype, gated=True)
     from test_layer_kernels import layer_case, split
     print("CASE chain walk, layer span", dtype, b, L, h, g, flush=True)
@@ -297,7 +378,7 @@ def test_layer_span(dtype, b, L, h, g):
     torch.testing.assert_close(y.float(), ref.reshape(b, L, -1).float(), rtol=2e-2, atol=2e-2)
 
 
-SPANS_TWO = [(4, 512, 128, 8), (3, 1216, 96, 8), (1, 2752, 96, 16), (3, 1472, 48, 8), (3, 1344, 96, 8)]
+SPANS_TWO = [(4, 512, 128, 8), (3, 1216, 96, 8), (1, 2752, 96, 16), (3, 1472, 48, 8), (3, 1344, 96, 8), (5, 1024, 48, 8)]
 
 
 @pytest.mark.gpu
@@ -427,9 +508,9 @@ def test_counted_waits(src, tmp_path):
             elif "f32" in src:
                 assert waits == {0: 0, 40: 0}, (name, waits)
             else:
-                gated = name.endswith("ELb1EEEvNS_13ChainScanArgsE")
+                gated = re.search(r"ELb[01]ELb([01])ELb[01]EEEvNS_13ChainScanArgsE$", name).group(1) == "1"
                 assert waits == {0: 0, 9: 0, 8 if gated else 4: 4}, (name, waits)
-    assert seen == {"ssd_chain_scan.hip": 16, "ssd_chain_scan_f32.hip": 4}[src]
+    assert seen == {"ssd_chain_scan.hip": 24, "ssd_chain_scan_f32.hip": 4}[src]
 
 
 def test_w_tiles():

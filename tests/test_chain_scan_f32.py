@@ -44,7 +44,7 @@ def case(b, L, h, g, N, seed):
 def test_plans():
     """Every shape of the GPU tests takes the walk (256 CUs): whole chains, two heads per workgroup."""
     for b, L, h, g, N, chunk in SHAPES + [(9, 256, 64, 8, 64, 64), (9, 256, 64, 8, 128, 64)]:
-        assert S.walk_plan(b, L, h, 64, N, g, chunk, torch.float32) == (1, L // 64, 2, False), (b, L, h, g, N)
+        assert S.walk_plan(b, L, h, 64, N, g, chunk, torch.float32) == (1, L // 64, 2, False, False), (b, L, h, g, N)
     assert S.walk_plan(8, 192, 64, 64, 64, 4, 64, torch.float32) is None   # one workgroup per CU
     assert S.walk_plan(9, 192, 64, 64, 64, 64, 64, torch.float32) is None  # one head per group
 

@@ -51,7 +51,7 @@ class SSDDims(ctypes.Structure):
 
 
 class SSDWalkPlan(ctypes.Structure):
-    _fields_ = [(n, ctypes.c_int64) for n in ("segments", "steps", "heads", "linked")]
+    _fields_ = [(n, ctypes.c_int64) for n in ("segments", "steps", "heads", "linked", "hilo")]
 
 
 class SSDEpilogue(ctypes.Structure):

@@ -444,10 +444,14 @@ ssd::ChainScanPlan chain_shape_plan(const ssd_dims* d, int dtype, bool gated, si
   const ssd::ChainScanPlan none{0, 0, false};
   const bool f32 = dtype == SSD_DTYPE_F32;
   if ((f32 && gated) || d->headdim != 64 || (f32 ? d->dstate != 64 && d->dstate != 128 : d->dstate != 128)) return none;
-  const ssd::ChainScanPlan plan =
+  ssd::ChainScanPlan plan =
       f32 ? ssd::chain_scan_f32_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, d->dstate)
           : ssd::chain_scan_plan(d->batch, d->seqlen / 64, d->nheads, d->ngroups, gated);
   if (plan.nseg == 0 || chain_ws(d, dtype, plan.nseg).total > ws_bytes) return none;
+  // S reaches the off-diagonal product as exactly as on the stage kernels: as
+  // f16 rows with a scale each where those hand it over so (handover_format),
+  // else (chunk 128, and the gate at 64 / 128) as a hi + lo pair
+  if (!f32) plan.hilo = d->chunk != 256 && (gated || !f16s_small_shape(d));
   return plan;
 }
 
@@ -461,7 +465,14 @@ ssd::ChainScanPlan chain_plan(const ssd_dims* d, int dtype, const int64_t x_stri
   for (int64_t st : {x_strides[1], b_strides[1], c_strides[1], dt_strides ? dt_strides[1] : 0})
     if (st > (1 << 23)) return none;
   if (y_strides[1] > (1 << 23) || (epi && epi->z_strides[1] > (1 << 23))) return none;
-  return chain_shape_plan(d, dtype, epi != nullptr, ws_bytes);
+  ssd::ChainScanPlan plan = chain_shape_plan(d, dtype, epi != nullptr, ws_bytes);
+  // the chunk-256 chunk_scan, which reads f16 rows, takes 32-bit strides only
+  if (dtype != SSD_DTYPE_F32)
+    for (int k = 0; k < 3; ++k)
+      for (int64_t st : {x_strides[k], b_strides[k], c_strides[k], dt_strides ? dt_strides[k] : 0, y_strides[k],
+                         epi ? epi->z_strides[k] : 0})
+        if (st > INT_MAX && d->chunk == 256) plan.hilo = true;
+  return plan;
 }
 
 int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan, CumsumArgs k1, const void* x, const int64_t x_strides[4],
@@ -492,7 +503,7 @@ int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan,
   p.sdh = dt ? dt_strides[2] : 0;
   p.acs = k1.acs;
   p.cb = reinterpret_cast<float*>(ws + w.cb);
-  p.ct = ws + w.ct;
+  p.ct = plan.hilo ? nullptr : ws + w.ct;
   p.cscale = reinterpret_cast<float*>(ws + w.cscale);
   p.init = initial_states;
   p.final_state = final_states;
@@ -516,6 +527,7 @@ int run_chain_scan(const ssd_dims* d, int dtype, const ssd::ChainScanPlan& plan,
   p.nseg = plan.nseg;
   p.seg_len = plan.seg_len;
   p.wide = plan.wide;
+  p.hilo = plan.hilo;
   p.linked = ssd::chain_scan_linked(plan.nseg, in_place(d, initial_states, final_states));
   const int n = (int)d->dstate;
   const bool f32 = dtype == SSD_DTYPE_F32;
@@ -728,12 +740,12 @@ int ssd_forward_plan(const ssd_dims* d, int dtype, int state_dtype, int gated, i
   const int rc = check_dims_impl(d, dtype);
   if (rc) return rc;
   if (!out) return SSD_ERR_NULL_POINTER;
-  *out = ssd_walk_plan{0, 0, 0, 0};
+  *out = ssd_walk_plan{0, 0, 0, 0, 0};
   if (state_dtype != SSD_DTYPE_F32) return SSD_OK;
   const ssd_dims e = gated ? layer_core_dims(d, dtype) : forward_dims(d, dtype, state_dtype);
   if (!gated && small_forward(&e, state_dtype)) return SSD_OK;
   const ssd::ChainScanPlan plan = chain_shape_plan(&e, dtype, gated != 0, ws_layout(&e, state_dtype).total);
-  if (plan.nseg > 0) *out = ssd_walk_plan{plan.nseg, plan.seg_len, plan.wide ? 4 : 2, ssd::chain_scan_linked(plan.nseg, in_place != 0)};
+  if (plan.nseg > 0) *out = ssd_walk_plan{plan.nseg, plan.seg_len, plan.wide ? 4 : 2, ssd::chain_scan_linked(plan.nseg, in_place != 0), plan.hilo};
   return SSD_OK;
 }
 

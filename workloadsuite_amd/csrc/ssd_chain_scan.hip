@@ -64,15 +64,21 @@ __device__ __forceinline__ f32x16 mma32(f16x8 a, f16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-template <typename T, int HPW, bool HAS_DT, bool EPI>
+// HILO: S goes into the off-diagonal product as a hi + lo pair of the input type,
+// one product each (f16 pairs of the scaled rows; bf16, whose exponents are f32's,
+// of the values as they are, with C as it lies).
+template <typename T, int HPW, bool HAS_DT, bool EPI, bool HILO>
 __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs p) {
   constexpr int NW = 2 * HPW;
-  constexpr bool kCT = !std::is_same<T, f16>::value;  // C from chain_prep's f16 rows
+  constexpr bool kF16 = std::is_same<T, f16>::value;
+  constexpr bool kCT = !kF16 && !HILO;   // C from chain_prep's f16 rows
+  constexpr bool kRows = kF16 || !HILO;  // S as f16 rows with a scale each
+  typedef typename std::conditional<HILO, T, f16>::type E;  // of the off-diagonal operands
   constexpr int NX = 4 + (EPI ? 4 : 0);  // x copies and z loads left in flight at the first barrier
   constexpr int NY = 5 + 4;              // C.B^T loads and y stores left in flight at the second
   constexpr int DPW = 16 / NW;         // B (C) copies per wave
   __shared__ __attribute__((aligned(1024))) T bs[kQ * kN];
-  __shared__ __attribute__((aligned(1024))) f16 cl[kQ * kN];
+  __shared__ __attribute__((aligned(1024))) E cl[kQ * kN];
   __shared__ __attribute__((aligned(1024))) T xs[HPW * 2][kQ * kP];
   __shared__ __attribute__((aligned(1024))) T wl[HPW][kWBlocks * 64 * 8];
   // per head: Acs, dt and C row scales of the step's tokens; per wave: their
@@ -81,7 +87,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
   __shared__ __attribute__((aligned(256))) float dl[HAS_DT ? HPW : 1][HAS_DT ? kQ : 4];
   __shared__ __attribute__((aligned(256))) float csl[kCT ? HPW : 1][kCT ? kQ : 4];
   __shared__ __attribute__((aligned(256))) float wt[NW][kQ];
-  __shared__ __attribute__((aligned(128))) float rsl[NW][32];
+  __shared__ __attribute__((aligned(128))) float rsl[kRows ? NW : 1][32];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -270,11 +276,11 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     const float a_own = ab[lane];
     int co = coff;
     if constexpr (EPI) asm volatile("" : "+v"(co));  // (the eight addresses, kept over the steps, would not fit the registers)
-    auto read_c = [&, coff = co](f16x8 (&cf)[2], int kb) __attribute__((always_inline)) {
+    auto read_c = [&, coff = co](frag8<E> (&cf)[2], int kb) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) cf[t] = *reinterpret_cast<const f16x8*>(cl + (coff ^ (16 * kb)) + 32 * t * kN);
+      for (int t = 0; t < 2; ++t) cf[t] = *reinterpret_cast<const frag8<E>*>(cl + (coff ^ (16 * kb)) + 32 * t * kN);
     };
-    f16x8 cf[2][2];
+    frag8<E> cf[2][2];
     read_c(cf[0], 0);
     // operands of this wave's five W tiles
     constexpr int kDI[5] = {0, 0, 1, 0, 2}, kTI[5] = {0, 0, 1, 0, 0};
@@ -290,17 +296,20 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     __builtin_amdgcn_sched_barrier(0);
     // S as f16 rows: the row's largest magnitude over the tiles, then over the two halves
     // (four independent chains, two values an instruction)
-    float mx[4];
+    float m = 0.f;
+    if constexpr (kRows) {
+      float mx[4];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) mx[nt] = __builtin_elementwise_maximum(fabsf(st[nt][0]), fabsf(st[nt][1]));
+      for (int nt = 0; nt < 4; ++nt) mx[nt] = __builtin_elementwise_maximum(fabsf(st[nt][0]), fabsf(st[nt][1]));
 #pragma unroll
-    for (int j = 2; j < 16; j += 2)
+      for (int j = 2; j < 16; j += 2)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        mx[nt] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(st[nt][j]), fabsf(st[nt][j + 1])), mx[nt]);
-    float m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx[0], mx[1]), __builtin_elementwise_maximum(mx[2], mx[3]));
-    const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    m = nn_max(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+        for (int nt = 0; nt < 4; ++nt)
+          mx[nt] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(st[nt][j]), fabsf(st[nt][j + 1])), mx[nt]);
+      m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx[0], mx[1]), __builtin_elementwise_maximum(mx[2], mx[3]));
+      const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+      m = nn_max(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+    }
     const float aq = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(a_own), 63));
     const float dec = __builtin_amdgcn_exp2f(aq * kLog2e);
     {
@@ -313,21 +322,33 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
-    const int e = m > 0.f ? min(max(__builtin_amdgcn_frexp_expf(m) - 15, -100), 100) : 0;
-    const float sc = __builtin_ldexpf(1.f, -e);
-    if (hl == 0) rsl[wave][r] = __builtin_ldexpf(1.f, e);
-    // (scaled and rounded by one v_fma_mixlo / mixhi per value: the opaque -0
-    // addend keeps the compiler from making it a product and a conversion)
-    float nz = -0.f;
-    asm("" : "+v"(nz));
-    auto f16_rows = [&](int kb) __attribute__((always_inline)) {
-      f16x8 v;
+    float sc = 1.f, nz = -0.f;
+    if constexpr (kRows) {
+      const int e = m > 0.f ? min(max(__builtin_amdgcn_frexp_expf(m) - 15, -100), 100) : 0;
+      sc = __builtin_ldexpf(1.f, -e);
+      if (hl == 0) rsl[wave][r] = __builtin_ldexpf(1.f, e);
+      // (scaled and rounded by one v_fma_mixlo / mixhi per value: the opaque -0
+      // addend keeps the compiler from making it a product and a conversion)
+      asm("" : "+v"(nz));
+    }
+    frag8<E> sf[2], sl[2];
+    auto operand_s = [&](int kb) __attribute__((always_inline)) {
+      const f32x16& v = st[kb >> 1];
+      const int j0 = 8 * (kb & 1);
+      if constexpr (kRows) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = (f16)__builtin_fmaf(st[kb >> 1][8 * (kb & 1) + j], sc, nz);
-      return v;
+        for (int j = 0; j < 8; ++j) {
+          sf[kb & 1][j] = (f16)__builtin_fmaf(v[j0 + j], sc, nz);
+          if constexpr (HILO) sl[kb & 1][j] = (f16)__builtin_fmaf(v[j0 + j], sc, -(float)sf[kb & 1][j]);
+        }
+      } else {
+        f32x4 a, b2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = v[j0 + j], b2[j] = v[j0 + 4 + j];
+        split_f32<T>(a, b2, sf[kb & 1], sl[kb & 1]);
+      }
     };
-    f16x8 sf[2];
-    sf[0] = f16_rows(0);
+    operand_s(0);
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) {
       if (kb < 7) read_c(cf[(kb + 1) & 1], kb + 1);
@@ -344,7 +365,11 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t) acc[t] = mma32(sf[kb & 1], cf[kb & 1][t], acc[t]);
-      if (kb < 7) sf[(kb + 1) & 1] = f16_rows(kb + 1);
+      if constexpr (HILO) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = mma32(sl[kb & 1], cf[kb & 1][t], acc[t]);
+      }
+      if (kb < 7) operand_s(kb + 1);
       // the state's decay, its value entering the step being taken
 #pragma unroll
       for (int j = 0; j < 8; ++j) st[kb >> 1][8 * (kb & 1) + j] *= dec;
@@ -373,14 +398,16 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const f32x4 rs = *reinterpret_cast<const f32x4*>(&rsl[wave][8 * k + 4 * hl]);
+      f32x4 rs = f32x4{1.f, 1.f, 1.f, 1.f};
+      if constexpr (kRows) rs = *reinterpret_cast<const f32x4*>(&rsl[wave][8 * k + 4 * hl]);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) acc[t][4 * k + jj] *= rs[jj] * ev[t];
+        for (int jj = 0; jj < 4; ++jj) acc[t][4 * k + jj] *= kRows ? rs[jj] * ev[t] : ev[t];
     }
     if (c < last) bg += bst;
     if (c + 1 < last) xg += xst;
+    accesses_before_wait();
     vm_wait<NX>();
     __syncthreads();
 
@@ -499,6 +526,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
       store16_g(yr, yv, __builtin_bit_cast(f32x4, oa));
       store16_g(yr + 16 * p.syl, yv, __builtin_bit_cast(f32x4, ob));
     }
+    accesses_before_wait();
     vm_wait<NY>();
     __syncthreads();
   }
@@ -688,25 +716,25 @@ hipError_t launch_state_t(const ChainScanArgs& a, hipStream_t stream) {
   return launch_state_passing(sp, SSD_DTYPE_F32, stream);
 }
 
-template <typename T, int HPW, bool HAS_DT, bool EPI>
+template <typename T, int HPW, bool HAS_DT, bool EPI, bool HILO>
 hipError_t launch_scan_t(const ChainScanArgs& a, hipStream_t stream) {
   const int64_t grid = (int64_t)a.batch * a.nseg * (a.nheads / HPW);
   if (grid > INT32_MAX) return hipErrorInvalidValue;
-  auto kern = chain_scan_kernel<T, HPW, HAS_DT, EPI>;
+  auto kern = chain_scan_kernel<T, HPW, HAS_DT, EPI, HILO>;
   kern<<<dim3((unsigned)grid), dim3(128 * HPW), 0, stream>>>(a);
   return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, bool HILO>
 hipError_t launch_t(const ChainScanArgs& a, hipStream_t stream) {
   const int hpg = a.nheads / a.ngroups;
   if (hpg % 2 != 0) return hipErrorInvalidValue;
   hipError_t e = hipSuccess;
   if (a.nseg > 1) e = hpg % 4 == 0 ? launch_state_t<T, 4>(a, stream) : launch_state_t<T, 2>(a, stream);
   if (e != hipSuccess) return e;
-  if (!a.z) return a.dt ? launch_scan_t<T, 2, true, false>(a, stream) : launch_scan_t<T, 2, false, false>(a, stream);
+  if (!a.z) return a.dt ? launch_scan_t<T, 2, true, false, HILO>(a, stream) : launch_scan_t<T, 2, false, false, HILO>(a, stream);
   if (!a.dt) return hipErrorInvalidValue;  // (the gate belongs to the layer, whose dt is always there)
-  return a.wide ? launch_scan_t<T, 4, true, true>(a, stream) : launch_scan_t<T, 2, true, true>(a, stream);
+  return a.wide ? launch_scan_t<T, 4, true, true, HILO>(a, stream) : launch_scan_t<T, 2, true, true, HILO>(a, stream);
 }
 
 }  // namespace
@@ -775,8 +803,8 @@ hipError_t launch_chain_prep(const ChainScanArgs& a, const CumsumArgs& ca, int d
 }
 
 hipError_t launch_chain_scan(const ChainScanArgs& a, int dtype, hipStream_t stream) {
-  if (dtype == SSD_DTYPE_BF16) return launch_t<bf16>(a, stream);
-  if (dtype == SSD_DTYPE_F16) return launch_t<f16>(a, stream);
+  if (dtype == SSD_DTYPE_BF16) return a.hilo ? launch_t<bf16, true>(a, stream) : launch_t<bf16, false>(a, stream);
+  if (dtype == SSD_DTYPE_F16) return a.hilo ? launch_t<f16, true>(a, stream) : launch_t<f16, false>(a, stream);
   return hipErrorInvalidValue;
 }
 

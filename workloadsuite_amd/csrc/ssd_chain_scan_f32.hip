@@ -289,6 +289,7 @@ __global__ __launch_bounds__(64 * kWaves, N == 64 ? 3 : 2) void chain_scan_f32_k
       __builtin_amdgcn_sched_barrier(0);
     }
     yg += (int64_t)kStep * p.syl;
+    accesses_before_wait();
     vm_wait<NY>();
     __syncthreads();
   }

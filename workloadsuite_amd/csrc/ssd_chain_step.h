@@ -58,6 +58,11 @@ __device__ __forceinline__ void store16_g(void* base, uint32_t v, f32x4 d) {
   *(gptr)((char __attribute__((address_space(1)))*)base + v) = d;
 }
 
+// In front of a counted wait (vm_wait) that relies on loads the compiler issued
+// before it: without a store or an access it knows nothing of in between, they may
+// end up behind the wait and its barrier, next to their use.
+__device__ __forceinline__ void accesses_before_wait() { asm volatile("" ::: "memory"); }
+
 // The causal tiles (row tile t of l, column tile s of s, s <= t) in pairs 2 m +
 // w, one for each wave of a head: (t, s) = (kT[m] + kDT[m] w, kS[m] + kDS[m] w).
 // Pairs 0 and 1 are the diagonal ones.
@@ -89,6 +94,7 @@ __device__ __forceinline__ void chain_prep_body(const ChainScanArgs& p, int bcg,
     cb[k * 64] = d;
   }
   if constexpr (std::is_same<T, bf16>::value) {
+    if (!p.ct) return;  // (S as a hi + lo pair: the walk takes C as it lies)
     // each row as f16 times 2^-e, its largest element in [2^14, 2^15) (bf16
     // values then convert exactly down to 2^-24 of it), in operand order:
     // piece 4 kc + g holds n = 32 kc + 4 g .. + 3 and 32 kc + 16 + 4 g .. + 3

@@ -103,6 +103,31 @@ __device__ __forceinline__ void split_weighted(const frag8<T>& b, f32x4 w0, f32x
   }
 }
 
+// Eight f32 values as a hi + lo pair of T: hi = T(v), lo = T(v - hi) (exact
+// residuals; pairs converted together, hi's f32 value from its bits for bf16).
+template <typename T>
+__device__ __forceinline__ void split_f32(f32x4 a, f32x4 b, frag8<T>& hi, frag8<T>& lo) {
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const float v0 = j < 4 ? a[j] : b[j - 4], v1 = j < 4 ? a[j + 1] : b[j - 3];
+    const t2 h = __builtin_convertvector((f32x2{v0, v1}), t2);
+    f32x2 hf;
+    if constexpr (std::is_same<T, bf16>::value) {
+      const uint32_t hu = __builtin_bit_cast(uint32_t, h);
+      hf = f32x2{__uint_as_float(hu << 16), __uint_as_float(hu & 0xffff0000u)};
+    } else {
+      hf = __builtin_convertvector(h, f32x2);
+    }
+    const t2 l = __builtin_convertvector((f32x2{v0 - hf[0], v1 - hf[1]}), t2);
+    hi[j] = h[0];
+    hi[j + 1] = h[1];
+    lo[j] = l[0];
+    lo[j + 1] = l[1];
+  }
+}
+
 // Larger of two non-negative floats (magnitudes, or maxima of magnitudes)
 // as an unsigned integer max of their bits: for non-negative IEEE values the
 // order of the bit patterns is the numeric order, so a finite result is

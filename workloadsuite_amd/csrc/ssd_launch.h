@@ -227,7 +227,7 @@ struct ChainScanArgs {
   int64_t sdb, sdl, sdh;
   const float* acs;       // [b, h, steps, 64] (K1 at chunk 64)
   float* cb;              // chain_prep: C.B^T tiles per (b, step, group)
-  void* ct;               // chain_prep, bf16 inputs: C as f16 rows
+  void* ct;               // chain_prep, bf16 inputs: C as f16 rows (null: not wanted)
   float* cscale;          // ... and their scales
   const float* init;      // optional [b, h, P, N]
   float* final_state;     // optional [b, h, P, N]
@@ -240,6 +240,7 @@ struct ChainScanArgs {
   int64_t szb = 0, szl = 0, szh = 0;
   int batch, nsteps, nheads, ngroups, nseg, seg_len;
   bool wide = false;      // epilogue: four heads per workgroup instead of two
+  bool hilo = false;      // S into the off-diagonal product as a hi + lo pair of the input type, not as f16 rows
   bool linked = false;    // state_passing forms the states entering the segments (chain_scan_linked)
 };
 // Up to this many segments, each workgroup of the scan forms its entering
@@ -253,7 +254,7 @@ inline bool chain_scan_linked(int nseg, bool in_place) { return nseg > kFoldSegs
 // not supported, or the stage kernels are as fast.
 struct ChainScanPlan {
   int nseg, seg_len;
-  bool wide;
+  bool wide, hilo = false;
 };
 ChainScanPlan chain_scan_plan(int64_t batch, int64_t steps, int64_t nheads, int64_t ngroups, bool epi);
 // bytes of cb / ct / cscale for `steps` = batch * nsteps * ngroups

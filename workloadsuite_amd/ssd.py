@@ -256,6 +256,7 @@ class WalkPlan(NamedTuple):
     steps: int     # 64-token steps per segment
     heads: int     # per workgroup
     linked: bool   # the states entering the segments come from a launch of their own
+    hilo: bool     # the state enters C.S as a hi + lo pair of the input type (else as f16 rows with a scale each)
 
 
 def walk_plan(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, dtype, state_dtype=torch.float32,
@@ -268,7 +269,7 @@ def walk_plan(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, dtype
     p = _lib.SSDWalkPlan()
     _lib.check(_lib.load().ssd_forward_plan(ctypes.byref(d), _DTYPES[dtype], _handover(state_format, dtype, state_dtype),
                                             int(gated), int(in_place), ctypes.byref(p)))
-    return WalkPlan(p.segments, p.steps, p.heads, bool(p.linked)) if p.segments else None
+    return WalkPlan(p.segments, p.steps, p.heads, bool(p.linked), bool(p.hilo)) if p.segments else None
 
 
 # ssd_forward's per-call host work, kept per layout: the ctypes dims and
