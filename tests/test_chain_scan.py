@@ -210,6 +210,28 @@ def test_strided_operands_match_contiguous_ones():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("b,L,h,g", [(3, 1216, 80, 1), (3, 1472, 48, 8), (2, 2496, 64, 8)])
+def test_growth_beyond_f32_over_a_segment(b, L, h, g):
+    """Log-decays of +0.4 over the first 256 tokens (a factor e^102) with x zero
+    there: no state exists yet, and the rest is as if the sequence began later.
+    (bf16: in f16 the weights of one 64-token block, up to e^25, are infinite.)"""
+    print("CASE chain walk, growth over a segment", b, L, h, g, flush=True)
+    dtype = torch.bfloat16
+    on_the_walk(b, L, h, g, dtype)
+    assert PLANS[b, L, h, g][0] > 1 and PLANS[b, L, h, g][1] > 4
+    X, A, B, C, dt, _ = case(dtype, b, L, h, g, seed=6)
+    A[:, :256] = 0.4
+    X[:, :256] = 0
+    hs = [0, h // 2, h - 1]
+    grp = [k // (h // g) for k in hs]
+    ref, fref = O.ssd_chunked(*(t[:, 256:] for t in (X[:, :, hs], A[:, :, hs], B[:, :, grp], C[:, :, grp])), 64,
+                              dt=dt[:, 256:, hs])
+    Y, final = S.ssd_forward(*(t.to(DEV) for t in (X, A, B, C)), 64, dt=dt.to(DEV), return_final_states=True)
+    check(Y[:, 256:, hs], final[:, hs], ref, fref)
+    assert (Y[:, :256] == 0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("what", ["x", "B", "C"])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("b,L,h,g", [(8, 384, 64, 4), (3, 1216, 80, 1)])

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-          for (int k = 0; k < 16; ++k) st[nt][k] = __builtin_fmaf(st[nt][k], dj, lo[nt][k]);
+          for (int k = 0; k < 16; ++k) st[nt][k] = __builtin_fmaf(st[nt][k] * dj, dj, lo[nt][k]);
       }
     }
   }
@@ -543,8 +543,9 @@ __global__ __launch_bounds__(128 * HPW, 2) void chain_scan_kernel(ChainScanArgs 
 }
 
 // The state at the end of every segment but the last, from a zero state, and
-// the segment's decay (one product per step): the scan's state update alone,
-// for chains too few to fill the GPU as one segment each.  A step here is
+// the square root of the segment's decay (of many tokens: where their log-decays
+// are positive the decay itself may lie beyond f32, and a state that is still
+// zero has to stay so): the scan's state update alone, for chains too few to fill the GPU as one segment each.  A step here is
 // shorter than the latency of HBM, so B and x are copied two steps ahead, into
 // a ring of three buffers; one barrier per step.
 template <typename T, int HPW, bool HAS_DT>
@@ -620,7 +621,7 @@ __global__ __launch_bounds__(128 * HPW, HPW == 4 ? 2 : 1) void chain_state_kerne
   for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) st[nt][j] = 0.f;
-  float dtot = 1.f;
+  float atot = 0.f;
   int bf = 0;
   const int q = i & 3, trow = 4 * hl + (i >> 2);
   int boff[4];
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(128 * HPW, HPW == 4 ? 2 : 1) void chain_state_kerne
     float wv = __builtin_amdgcn_exp2f((aq - a_own) * kLog2e);
     if constexpr (HAS_DT) wv *= dl[bf][wave][lane];
     wt[wave][lane] = wv;
-    dtot *= dec;
+    atot += aq;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) st[nt] *= dec;
     f32x4 w0 = read_wt(0), w1 = read_wt(1);
@@ -691,7 +692,7 @@ __global__ __launch_bounds__(128 * HPW, HPW == 4 ? 2 : 1) void chain_state_kerne
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       *reinterpret_cast<f32x4*>(fp + 32 * nt + 16 * (k >> 1) + 4 * (k & 1)) = f32x4{st[nt][4 * k], st[nt][4 * k + 1], st[nt][4 * k + 2], st[nt][4 * k + 3]};
-  if (w == 0 && lane == 0) p.seg_decay[((int64_t)b * p.nheads + h) * p.nseg + seg] = dtot;
+  if (w == 0 && lane == 0) p.seg_decay[((int64_t)b * p.nheads + h) * p.nseg + seg] = __builtin_amdgcn_exp2f(atot * (0.5f * kLog2e));
 }
 
 template <typename T, int HPW>
@@ -706,6 +707,7 @@ hipError_t launch_state_t(const ChainScanArgs& a, hipStream_t stream) {
   StatePassingArgs sp;
   sp.states = a.seg_states;
   sp.decay = a.seg_decay;
+  sp.root_decay = true;
   sp.init = a.init;
   sp.final_state = nullptr;
   sp.batch = a.batch;

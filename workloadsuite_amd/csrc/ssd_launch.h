@@ -65,6 +65,7 @@ struct StatePassingArgs {
   // (SSD_STATE_F16S, in place in the f32 layout; chunk-256 forward path only)
   int f16s = 0;
   float* sscale = nullptr;  // f16s: the row scales [b, c, h, P]
+  bool root_decay = false;  // decay holds the decays' square roots (plain f32 states only)
   // chains (b * nheads + h) [bh_begin, bh_begin + bh_count) only; bh_count 0: all
   int bh_begin = 0, bh_count = 0;
 };
@@ -232,7 +233,7 @@ struct ChainScanArgs {
   const float* init;      // optional [b, h, P, N]
   float* final_state;     // optional [b, h, P, N]
   float* seg_states;      // nseg > 1: the state entering each segment [b, nseg, h, P, N]
-  float* seg_decay;       // ... and the segments' decays [b, h, nseg]
+  float* seg_decay;       // ... and the square roots of the segments' decays [b, h, nseg]
   void* y;
   int64_t syb, syl, syh;  // y [b, L, h, P], 16-byte aligned rows
   const float* dskip = nullptr;  // epilogue (with z): y = (y + dskip[h] x) * silu(z)

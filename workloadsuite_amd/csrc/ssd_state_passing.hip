@@ -61,8 +61,9 @@ template <> struct StateIO<bf16> {
 // current kUnroll chunks' stores and FMAs, so each thread always has a batch
 // of loads in flight (two register batches used in turn: no copies between
 // them, which would wait for the loads).  load(c) returns chunk c's local
-// state, store(c, v) writes S_in[c] = v; dec[c] is chunk c's decay.
-template <int kUnroll = 8, typename V, typename LoadF, typename StoreF>
+// state, store(c, v) writes S_in[c] = v; dec[c] is chunk c's decay (ROOT: its
+// square root).
+template <int kUnroll = 8, bool ROOT = false, typename V, typename LoadF, typename StoreF>
 __device__ __forceinline__ V run_chain(int nchunks, const float* __restrict__ dec, V st, LoadF load,
                                        StoreF store) {
   V la[kUnroll], lb[kUnroll];
@@ -86,7 +87,7 @@ __device__ __forceinline__ V run_chain(int nchunks, const float* __restrict__ de
     for (int u = 0; u < kUnroll; ++u) {
       if (all || c0 + u < nchunks) {
         store(c0 + u, st);
-        st = st * d[u] + l[u];
+        st = (ROOT ? st * d[u] : st) * d[u] + l[u];
       }
     }
   };
@@ -110,7 +111,7 @@ __device__ __forceinline__ V run_chain(int nchunks, const float* __restrict__ de
   return st;
 }
 
-template <typename S>
+template <typename S, bool ROOT>
 __global__ __launch_bounds__(256) void state_passing_kernel(StatePassingArgs p) {
   const int64_t PN = (int64_t)p.headdim * p.dstate;
   const int vec_per_bh = (int)(PN / 4);
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(256) void state_passing_kernel(StatePassingArgs p) 
 
   f32x4 st = p.init ? *reinterpret_cast<const f32x4*>(p.init + (int64_t)bh * PN + 4 * (int64_t)v)
                     : f32x4{0.f, 0.f, 0.f, 0.f};
-  st = run_chain(
+  st = run_chain<8, ROOT>(
       p.nchunks, dec, st,
       [&](int c, auto nt) { return StateIO<S>::template load<decltype(nt)::value>(base + c * cstride); },
       [&](int c, f32x4 val) { StateIO<S>::store(base + c * cstride, val); });
@@ -320,6 +321,7 @@ hipError_t launch_state_passing(const StatePassingArgs& a, int state_dtype, hipS
   const int64_t all = (int64_t)a.batch * a.nheads;
   if (a.bh_begin < 0 || a.bh_count < 0 || a.bh_begin + (int64_t)a.bh_count > all) return hipErrorInvalidValue;
   const int64_t chains = a.bh_count > 0 ? a.bh_count : all - a.bh_begin;
+  if (a.root_decay && (a.f16s || a.split_dtype != 0 || state_dtype != SSD_DTYPE_F32)) return hipErrorInvalidValue;
   if (a.f16s) {
     // 8 states per thread (two 16-byte loads of f32 local states or one of f16
     // ones, one 16-byte f16 store per chunk) in batches of 2 chunks: 76 VGPRs.
@@ -356,9 +358,10 @@ hipError_t launch_state_passing(const StatePassingArgs& a, int state_dtype, hipS
   const int64_t blocks_per_bh = (PN / 4 + 255) / 256;
   const dim3 grid((unsigned)(chains * blocks_per_bh));
   if (state_dtype == SSD_DTYPE_F32) {
-    state_passing_kernel<float><<<grid, 256, 0, stream>>>(a);
+    if (a.root_decay) state_passing_kernel<float, true><<<grid, 256, 0, stream>>>(a);
+    else state_passing_kernel<float, false><<<grid, 256, 0, stream>>>(a);
   } else if (state_dtype == SSD_DTYPE_BF16) {
-    state_passing_kernel<bf16><<<grid, 256, 0, stream>>>(a);
+    state_passing_kernel<bf16, false><<<grid, 256, 0, stream>>>(a);
   } else {
     return hipErrorInvalidValue;
   }
