@@ -6,9 +6,11 @@
     python bench.py --layer [--steps K] [--warmup W]
     python bench.py --decode [--decode-batches 4,64,256]
 
-A step is one SSD forward (K1 cumsum and K0 chunk_prep in one launch -> K2
-chunk_state and K3 state_passing, one launch per (b, h) chain where that is
-faster -> K4 chunk_scan) over one batch of synthetic inputs already resident in HBM, at
+A step is one SSD forward (by default a walk along the (batch, head) chains where
+the library takes it, as at C3; with --state-format f16s or split, and elsewhere,
+the stage kernels: K1 cumsum and K0 chunk_prep in one launch -> K2 chunk_state and
+K3 state_passing, one launch per (b, h) chain where that is faster -> K4
+chunk_scan) over one batch of synthetic inputs already resident in HBM, at
 the Mamba-2-2.7B layer shape by default (C3: batch 4, seqlen 4096, 80 heads,
 head_dim 64, d_state 128, chunk 256, 1 group, bf16 X/B/C, fp32 A, final state
 returned).  Prints ONE JSON line.
@@ -22,7 +24,9 @@ the measurements before the timed region bring the GPU to its steady state.
 Kernel durations are measured live with HIP events on the
 stream the kernels run on (torch's current stream), and the dominant kernel's
 algorithmic bytes (or flops) per launch over that duration give
-``roofline.achieved``.  ``cpu_baseline`` times the CPU oracle's float32
+``roofline.achieved``.  A forward that is one chain walk (two to four launches
+without entry points of their own) or one launch is timed whole; its launches
+one by one are in profiles/ssd_chain_walk.md.  ``cpu_baseline`` times the CPU oracle's float32
 restatement of the reference einsum path on a bounded sample (one batch
 element of the same config) on this host's cores.
 
@@ -168,11 +172,23 @@ def end_to_end_model(cfg):
     return flops, byts
 
 
+def walk_profile(cfg, key):
+    """The line ``<key> chain_walk <config>: <n>`` of profiles/ssd_chain_walk.md (one whole forward), or None."""
+    path = os.path.join(ROOT, "profiles", "ssd_chain_walk.md")
+    start = f"{key} chain_walk {cfg.name}:"
+    for line in open(path) if os.path.exists(path) else ():
+        if line.startswith(start):
+            return int(line[len(start):].strip()), os.path.relpath(path, ROOT)
+    return None, None
+
+
 def profiled_traffic(cfg, kernel):
     """HBM bytes per launch of `kernel` as measured with rocprofv3 FETCH_SIZE /
     WRITE_SIZE (scaled by a copy of known size) and committed under
     profiles/ssd_forward_<config>.md as a line ``traffic_bytes_per_launch
     <kernel>: <bytes>``; (None, None) when there is no such measurement."""
+    if kernel == "chain_walk":
+        return walk_profile(cfg, "traffic_bytes_per_forward")
     path = os.path.join(ROOT, "profiles", f"ssd_forward_{cfg.name}.md")
     if not os.path.exists(path):
         return None, None
@@ -189,6 +205,8 @@ def profiled_mfma(cfg, kernel):
     profiles/ssd_forward_<config>.md in lines ``mfma_instructions_per_launch
     <kernel>: <n>`` and ``mfma_flops_per_instruction <kernel>: <f>``;
     None when there is no such measurement."""
+    if kernel == "chain_walk":
+        return walk_profile(cfg, "mfma_flops_per_forward")[0]
     path = os.path.join(ROOT, "profiles", f"ssd_forward_{cfg.name}.md")
     if not os.path.exists(path):
         return None
@@ -573,6 +591,14 @@ def main():
     if prep is None:
         del kfn["chunk_prep"]
     small = takes_small_path(kcfg, state_dtype)
+    walk = S.walk_plan(cfg.batch, cfg.seqlen, cfg.nheads, cfg.headdim, cfg.dstate, cfg.ngroups, cfg.chunk, cfg.dtype,
+                       state_dtype, args.state_format)
+    if walk is not None:
+        # the forward is a chain walk: timed whole, with the forward's minimum
+        # bytes and flops; the stage entry points are not what it runs
+        kfn = {"chain_walk": lambda: S.ssd_forward(X, A, B, C, cfg.chunk, initial_states=init,
+                                                   return_final_states=cfg.final_state, state_dtype=state_dtype,
+                                                   state_format=args.state_format)}
     if small:
         # the forward is one launch (ssd_small): time it, with the forward's
         # minimum bytes and flops; the four stages' entry points are not what
@@ -584,6 +610,7 @@ def main():
                          cb_in_scan=prep is None)
     f_min, b_min = end_to_end_model(cfg)
     model["ssd_small"] = dict(bytes=b_min, flops=f_min)
+    model["chain_walk"] = dict(bytes=b_min, flops=end_to_end_model(cfg.scaled(chunk=64))[0])  # 64-token steps
     kernels = {}
     pre_launches = 0
 
@@ -614,25 +641,6 @@ def main():
         fn()
         kernels[name] = kernel_entry(name, time_launches(fn, args.kernel_reps))
         pre_launches += 1 + args.kernel_reps
-    # the dominant stage kernel: K2 + K3 as the stage path runs them
-    # (chunk_state_passing), K4, K1 and K0 -- not the standalone chunk_state
-    # and state_passing rows, which stand in for it only as a breakdown.  (Where
-    # ssd_forward runs the chain walk, whose launches have no entry point of
-    # their own, these rows describe the stage kernels beside it.)
-    dom = max((k for k in kernels if k not in ("chunk_state", "state_passing")), key=lambda k: kernels[k]["ms"])
-    kd = kernels[dom]
-    if kd["bound"] == "hbm":
-        roof = {"bound": "hbm", "achieved": kd["GB_s"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                "frac": kd["hbm_frac"]}
-    else:
-        roof = {"bound": "mfma", "achieved": kd["TFLOP_s"], "peak": PEAK_TFLOPS[cfg.dtype], "unit": "TFLOP/s",
-                "frac": kd["mfma_frac"]}
-    roof["kernel"] = dom
-    if roof["bound"] == "mfma":
-        roof["flops_basis"] = "useful: causal triangle, C.B^T once per (batch, chunk, group)"
-        if "mfma_executed_frac" in kd:
-            roof["mfma_executed_frac"] = kd["mfma_executed_frac"]
-    roof["traffic"], roof["traffic_source"] = profiled_traffic(cfg, dom)
 
     # ---- K forwards timed one by one: per-step median / mean / p90 / p99 ----
     # A fresh process's first ~60 forwards run slower (C3, per 20 steps after
@@ -663,6 +671,30 @@ def main():
     ms_per_step = wall * 1e3 / args.steps
     tokens_per_s = cfg.tokens * args.steps / wall
 
+    if walk is not None:
+        # the row is the whole forward: its time is the timed region's, past the
+        # start-up ramp that the launches above run in
+        kernels["chain_walk"] = kernel_entry("chain_walk", dev_ms)
+    # the dominant kernel among those the forward runs: K2 + K3 as it runs them
+    # (chunk_state_passing), K4, K1 and K0 -- not the standalone chunk_state
+    # and state_passing rows, which stand in for it only as a breakdown; or the
+    # one row of a chain walk or one-launch forward
+    dom = max((k for k in kernels if k not in ("chunk_state", "state_passing")), key=lambda k: kernels[k]["ms"])
+    kd = kernels[dom]
+    if kd["bound"] == "hbm":
+        roof = {"bound": "hbm", "achieved": kd["GB_s"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
+                "frac": kd["hbm_frac"]}
+    else:
+        roof = {"bound": "mfma", "achieved": kd["TFLOP_s"], "peak": PEAK_TFLOPS[cfg.dtype], "unit": "TFLOP/s",
+                "frac": kd["mfma_frac"]}
+    roof["kernel"] = dom
+    if roof["bound"] == "mfma":
+        roof["flops_basis"] = ("useful: causal triangle of 64 tokens, C.B^T once per (batch, step, group)" if walk else
+                               "useful: causal triangle, C.B^T once per (batch, chunk, group)")
+        if "mfma_executed_frac" in kd:
+            roof["mfma_executed_frac"] = kd["mfma_executed_frac"]
+    roof["traffic"], roof["traffic_source"] = profiled_traffic(cfg, dom)
+
     roof_tps = min(PEAK_TFLOPS[cfg.dtype] * 1e12 / (f_min / cfg.tokens), PEAK_HBM_GBS * 1e9 / (b_min / cfg.tokens))
 
     out = {
@@ -680,10 +712,11 @@ def main():
         "data": "synthetic (seeded: X~N(0,1), B,C~N(0,1)/sqrt(N), A=-softplus(N(-2,1))*exp(N(0,.5)))",
         "config": {"workload": f"mamba2-ssd-forward {cfg.name}" + (" (Mamba-2-2.7B layer)" if cfg.name == "C3" else ""),
                    "batch": cfg.batch, "seqlen": cfg.seqlen, "nheads": cfg.nheads, "headdim": cfg.headdim,
-                   "dstate": cfg.dstate, "chunk": cfg.chunk, "chunk_run": run_chunk, "ngroups": cfg.ngroups,
+                   "dstate": cfg.dstate, "chunk": cfg.chunk, "chunk_run": 64 if walk else run_chunk, "ngroups": cfg.ngroups,
                    "inputs": f"{DTYPE_NAMES[cfg.dtype]} X/B/C, f32 A", "state_storage": args.state_dtype,
-                   "state_handover": split if isinstance(split, str) else ("split" if split is not None else None),
-                   "local_states": ("in LDS (one-launch forward)" if small else "f16 rows" if local_f16 else
+                   "state_handover": None if walk else split if isinstance(split, str) else ("split" if split is not None else None),
+                   "local_states": (f"in f32 registers (chain walk, {walk.segments} segment(s) of {walk.steps} 64-token steps)"
+                                    if walk else "in LDS (one-launch forward)" if small else "f16 rows" if local_f16 else
                                     "in registers (state chain)" if takes_state_chain(kcfg, split, state_dtype)
                                     else args.state_dtype),
                    "final_state": cfg.final_state, "initial_state": cfg.init_state},
