@@ -484,6 +484,35 @@ def test_config_full_size(name, batches, heads):
     assert_close(fg, fr, tol)
 
 
+STAGE_SIZES = [("C3", CONFIGS["C3"], [0, 3], [0, 41, 79]), ("C4", CONFIGS["C4"], [0], [0, 40, 79]),
+               ("R0", CONFIGS["R0"], [0, 7], [0, 17, 63, 64, 127]),
+               ("C5, one workgroup's worth per CU", CONFIGS["C5"].scaled(batch=8), [0, 7], [0, 13, 63]),
+               ("two whole chains per CU and a mixed plan", CONFIGS["C3"].scaled(batch=2, seqlen=2048, nheads=160), [1],
+                [0, 90, 159])]
+
+
+@pytest.mark.parametrize("name,cfg,batches,heads", STAGE_SIZES, ids=[s[0] for s in STAGE_SIZES])
+def test_stage_kernels_full_size(name, cfg, batches, heads):
+    """The stage kernels at full size (at C3, C4 and R0 the default runs a chain
+    walk; state_format "f16s", and in f32 a call of one two-chain workgroup per
+    CU, keep them): sampled heads against the oracle, Y and the final state."""
+    say("stage kernels", name, cfg)
+    fmt = None if cfg.dtype == torch.float32 else "f16s"
+    assert S.walk_plan(cfg.batch, cfg.seqlen, cfg.nheads, cfg.headdim, cfg.dstate, cfg.ngroups, cfg.chunk, cfg.dtype,
+                       state_format=fmt) is None
+    inp = to_dev(make_inputs(cfg, seed=0, device=DEV))
+    Y, final = S.ssd_forward(inp["X"], inp["A"], inp["B"], inp["C"], cfg.chunk, initial_states=inp["init"],
+                             return_final_states=True, state_format=fmt)
+    torch.cuda.synchronize()
+    assert torch.isfinite(Y).all() and torch.isfinite(final).all()
+    X, A, B, C, init = _slice_inputs(inp, batches, heads, cfg.ngroups, cfg.nheads)
+    Yr, fr = O.ssd_chunked(X, A, B, C, cfg.chunk, initial_states=init)
+    bs, hs = torch.tensor(batches), torch.tensor(heads)
+    tol = tolerance(cfg.dtype)
+    assert_close(Y.cpu()[bs][:, :, hs], Yr, tol)
+    assert_close(final.cpu()[bs][:, hs], fr, tol)
+
+
 def mr_regime_inputs(cfg, seed):
     """R0-shaped inputs in MR's own parameter regime (MR:61-63, 94, 102-103):
     A = -(1..h) (A_log = log(1..h)), dt = softplus(dt_raw - 4) with dt_raw,
@@ -522,19 +551,20 @@ def _check_mr_regime(Y, final, X, A, B, C, dt, heads, batches, block_len, ngroup
 def test_full_r0_forward_at_block_len_64_in_the_reference_regime():
     """R0 (batch 8, seqlen 2048, 128 heads, d_state 128, 8 groups, MR's
     block_len 64, f16) through ssd_forward with MR's own A and dt (see
-    mr_regime_inputs) and B / C per group, the form INTEGRATION's
-    "better" binding passes: the library runs it at chunk 256 (the
-    persistent kernels, in-chunk log-decay sums to ~-600).  Sampled heads
-    of every group on two batches against the float64 oracle at block_len
-    64, 2e-2, Y and the final state."""
+    mr_regime_inputs) and B / C per group, the form that passes them without
+    repeats: as the library runs it (a chain walk in 64-token steps), and on the
+    stage kernels, which take it at chunk 256 (the persistent kernels, in-chunk
+    log-decay sums to ~-600).  Sampled heads of every group on two batches
+    against the float64 oracle at block_len 64, 2e-2, Y and the final state."""
     cfg = CONFIGS["R0"]
     say("R0 forward, MR regime", cfg)
     X, A, B, C, dt = mr_regime_inputs(cfg, seed=21)
     assert S.forward_chunk(cfg.batch, cfg.seqlen, cfg.nheads, cfg.headdim, cfg.dstate, cfg.ngroups, 64,
                            torch.float16) == 256
-    Y, final = S.ssd_forward(X, A, B, C, 64, dt=dt, return_final_states=True)
-    torch.cuda.synchronize()
-    _check_mr_regime(Y, final, X, A, B, C, dt, R0_HEADS, [0, 7], 64, cfg.ngroups, cfg.nheads)
+    for fmt in (None, "f16s"):
+        Y, final = S.ssd_forward(X, A, B, C, 64, dt=dt, return_final_states=True, state_format=fmt)
+        torch.cuda.synchronize()
+        _check_mr_regime(Y, final, X, A, B, C, dt, R0_HEADS, [0, 7], 64, cfg.ngroups, cfg.nheads)
 
 
 def test_full_r0_ssd_core_on_the_block_64_kernels_in_the_reference_regime():
@@ -579,12 +609,12 @@ def forward_by_kernels(X, A, B, C, Q, dt=None, initial_states=None):
 def test_full_size_chunk_invariance_and_state_linearity(name):
     """Size-independent properties of the whole forward at the full config
     size (the oracle is too slow there): the chunked SSD computes one linear
-    recurrence whatever the chunk length (MR:152-161), so the chunk-256
-    persistent path (state chain, chunk_scan's persistent kernel) and the
-    chunk-64 kernels agree; and Y is linear in the initial state,
-    Y(X, S0) = Y(X, 0) + Y(0, S0), as is the final state.  Tolerances are the
-    16-bit one relative to each output's scale (every Y is rounded to bf16
-    once)."""
+    recurrence whatever the chunk length (MR:152-161), so the default (a chain
+    walk in segments), the chunk-256 persistent path that state_format "f16s"
+    keeps (state chain, chunk_scan's persistent kernel) and the chunk-64 kernels
+    agree; and Y is linear in the initial state, Y(X, S0) = Y(X, 0) + Y(0, S0),
+    as is the final state.  Tolerances are the 16-bit one relative to each
+    output's scale (every Y is rounded to bf16 once)."""
     cfg = CONFIGS[name]
     say("full-size properties", name)
     inp = to_dev(make_inputs(cfg, seed=3, device=DEV))
@@ -592,8 +622,9 @@ def test_full_size_chunk_invariance_and_state_linearity(name):
     gen = torch.Generator(device=DEV).manual_seed(4)
     S0 = 0.1 * torch.randn(cfg.batch, cfg.nheads, cfg.headdim, cfg.dstate, device=DEV, generator=gen)
     Y256, f256 = S.ssd_forward(X, A, B, C, 256, return_final_states=True)
-    # ssd_forward itself runs these 16-bit shapes at chunk 256 for any block
-    # length: the chunk-64 kernels one by one (f32-state chain, 16-bit chunk_scan)
+    Ys, fs = S.ssd_forward(X, A, B, C, 256, return_final_states=True, state_format="f16s")
+    # ssd_forward runs the stage kernels of these 16-bit shapes at chunk 256 for any
+    # block length: the chunk-64 kernels one by one (f32-state chain, 16-bit chunk_scan)
     Y64, f64 = forward_by_kernels(X, A, B, C, 64)
     Yi, fi = S.ssd_forward(X, A, B, C, 256, initial_states=S0, return_final_states=True)
     Y0, f0 = S.ssd_forward(torch.zeros_like(X), A, B, C, 256, initial_states=S0, return_final_states=True)
@@ -602,6 +633,8 @@ def test_full_size_chunk_invariance_and_state_linearity(name):
     scale = Y256.float().abs().max().item()
     fscale = f256.abs().max().item()
     assert torch.isfinite(Y256).all() and torch.isfinite(f256).all()
+    assert_close(Ys, Y256.float(), tol, atol=tol * scale)
+    assert_close(fs, f256, tol, atol=tol * fscale)
     assert_close(Y64, Y256.float(), tol, atol=tol * scale)
     assert_close(f64, f256, tol, atol=tol * fscale)
     assert_close(Yi, Y256.float() + Y0.float(), tol, atol=tol * scale)
@@ -609,16 +642,19 @@ def test_full_size_chunk_invariance_and_state_linearity(name):
 
 
 def test_long_context_weak_decay_recurrence():
-    """C4 shape with A scaled by 1e-3: 256 chunks of carried state dominate."""
+    """C4 shape with A scaled by 1e-3: 1024 steps (256 chunks) of carried state
+    dominate, in the default's chain walk and on the stage kernels."""
     cfg = CONFIGS["C4"]
     say("C4 weak decay")
     inp = to_dev(make_inputs(cfg, seed=1, device=DEV, a_scale=1e-3))
-    Y, final = S.ssd_forward(inp["X"], inp["A"], inp["B"], inp["C"], cfg.chunk, return_final_states=True)
     X, A, B, C, _ = _slice_inputs(inp, [0], [5, 66], 1, cfg.nheads)
     Yr, fr = O.ssd_chunked(X, A, B, C, cfg.chunk)
     hs = torch.tensor([5, 66])
-    assert_close(Y.cpu()[:, :, hs], Yr, 2e-2)
-    assert_close(final.cpu()[:, hs], fr, 2e-2)
+    for fmt in (None, "f16s"):
+        Y, final = S.ssd_forward(inp["X"], inp["A"], inp["B"], inp["C"], cfg.chunk, return_final_states=True,
+                                 state_format=fmt)
+        assert_close(Y.cpu()[:, :, hs], Yr, 2e-2)
+        assert_close(final.cpu()[:, hs], fr, 2e-2)
 
 
 # ---------------------------------------------------------------------------
@@ -740,7 +776,8 @@ def _random_cases(n, seed=11):
 def test_random_shapes_vs_oracle(k, dtype, Q, N, g, h, b, nc, use_dt, use_init):
     """Seeded random shapes (dtype, chunk, d_state, groups, heads, batch,
     chunks, dt, initial state) through ssd_forward against the chunked
-    oracle, Y and the final state."""
+    oracle, Y and the final state; where that is a chain walk (the shapes of
+    320 chains), the stage kernels' mixed plan too."""
     say("random", k, dtype, Q, N, g, h, b, nc, use_dt, use_init)
     cfg = CONFIGS["C2"].scaled(batch=b, seqlen=Q * nc, nheads=h, dstate=N, chunk=Q, ngroups=g, dtype=dtype,
                                init_state=use_init)
@@ -760,6 +797,11 @@ def test_random_shapes_vs_oracle(k, dtype, Q, N, g, h, b, nc, use_dt, use_init):
     tol = tolerance(dtype)
     assert_close(Y, Yr, tol)
     assert_close(final, fr, tol)
+    if S.walk_plan(b, Q * nc, h, 64, N, g, Q, dtype) is not None:
+        Y, final = S.ssd_forward(d["X"], d["A"], d["B"], d["C"], Q, dt=None if dt is None else dt.to(DEV),
+                                 initial_states=d["init"], return_final_states=True, state_format="f16s")
+        assert_close(Y, Yr, tol)
+        assert_close(final, fr, tol)
 
 
 def _sweep_cases(n, seed=2024):

@@ -205,7 +205,8 @@ def test_model_matches_layer_oracle(cfg):
     """mr_init keeps the module's own initialisation (MR:58-66: default
     nn.Linear / nn.Conv1d weights, A_log = log(1..h), dt_bias = -4, D = 1);
     the other cases spread A and the gates wider.  L = 512 with block_len 64
-    runs the core at chunk 256, compared with the oracle at block_len 64."""
+    runs the core at chunk 256 (too few chain steps for a walk), compared with the
+    oracle at block_len 64."""
     say("layer", cfg)
     cfg = dict(cfg)
     L, b, mr_init = cfg.pop("L"), cfg.pop("b"), cfg.pop("mr_init", False)
@@ -252,10 +253,9 @@ def test_full_r0_layer_span_matches_oracle_with_reference_init():
     128 heads, d_state 128, 8 groups, block_len 64; MR:209-221) with the
     module's own initialisation: A = -(1..128), dt = softplus(dt_raw - 4),
     D = 1 (MR:61-63, 94), so in-chunk cumulative log-decays reach ~-600.  The
-    core runs at chunk 256 (1,024 chains: the whole-chain plan, and the
-    epilogue chunk_scan reading chunk_prep's 16-bit C.B^T).  The span's output
-    (out_proj's input) is compared on sampled batches and heads -- every group
-    is covered -- with the float64 oracle at MR's block_len 64, 2e-2."""
+    core runs as a chain walk (1,024 whole chains, four heads per workgroup).  The
+    span's output (out_proj's input) is compared on sampled batches and heads --
+    every group is covered -- with the float64 oracle at MR's block_len 64, 2e-2."""
     say("R0 full size, MR init")
     torch.manual_seed(0)
     layer = ML.SSDLayer(2048, 128, 128, 64, 8, block_len=64, conv_kernel=4).to(DEV).eval()
@@ -272,6 +272,7 @@ def test_full_r0_layer_span_matches_oracle_with_reference_init():
         y_mod = layer(u)
     torch.cuda.synchronize()
     assert y.shape == (b, L, h * P) and torch.isfinite(y).all() and torch.isfinite(y_mod).all()
+    assert S.walk_plan(b, L, h, P, N, g, 64, torch.float16, gated=True) == (1, L // 64, 4, False, False)
     heads = [0, 1, 17, 40, 63, 64, 90, 100, 127]   # groups 0, 0, 1, 2, 3, 4, 5, 6, 7
     bs = torch.tensor([0, 7])
     cpu = lambda t: t[bs].cpu()  # noqa: E731
@@ -282,3 +283,31 @@ def test_full_r0_layer_span_matches_oracle_with_reference_init():
     # the module's forward is that span followed by out_proj
     with torch.inference_mode():
         torch.testing.assert_close(y_mod, layer.out_proj(y), rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.gpu
+def test_full_size_layer_span_on_the_stage_kernels():
+    """The same span and regime with 15 heads per group, which no walk takes: the
+    core runs at chunk 256 (960 chains: the whole-chain plan, and the epilogue
+    chunk_scan reading chunk_prep's 16-bit C.B^T).  Sampled heads of every group
+    against the float64 oracle at block_len 64, 2e-2."""
+    say("full size, MR init, stage kernels")
+    torch.manual_seed(0)
+    h, g, N, P = 120, 8, 128, 64
+    layer = ML.SSDLayer(1920, h, N, P, g, block_len=64, conv_kernel=4).to(DEV).eval()
+    u = torch.randn(8, 2048, 1920, device=DEV, dtype=torch.float16, generator=torch.Generator(device=DEV).manual_seed(1))
+    b, L = u.shape[:2]
+    assert S.walk_plan(b, L, h, P, N, g, 64, torch.float16, gated=True) is None
+    with torch.inference_mode():
+        x, z, B, C, dt = torch.split(layer.in_proj(layer.norm(u)), [h * P, h * P, g * N, g * N, h], dim=-1)
+        Bv, Cv = B.view(b, L, g, N), C.view(b, L, g, N)
+        y = S.ssd_layer(x, z, Bv, Cv, dt, layer.conv1d.weight, layer.conv1d.bias, layer.dt_bias, layer.A_log,
+                        layer.D, 64, h)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y).all()
+    heads = [0, 14, 15, 31, 59, 60, 75, 104, 119]
+    bs = torch.tensor([0, 7])
+    cpu = lambda t: t[bs].cpu()  # noqa: E731
+    ref = _span_oracle(cpu(x), cpu(z), cpu(Bv), cpu(Cv), cpu(dt), layer, heads, 64)
+    ch = torch.cat([torch.arange(hh * P, (hh + 1) * P) for hh in heads])
+    torch.testing.assert_close(y[bs].cpu()[..., ch].double(), ref, rtol=2e-2, atol=2e-2)
