@@ -88,8 +88,11 @@ extern "C" {
  * F16S_LOCAL; the chain keeps them in f32 registers.  So the forward's last
  * bits depend on the launch plan, which depends on batch x heads and the
  * device's CU count: results are not bitwise invariant to batch slicing.
- * state_dtype SPLIT (at chunk 256) keeps every local state in f32.  (None of
- * this concerns the forwards that run as a chain walk, see ssd_forward.) */
+ * state_dtype SPLIT (at chunk 256) keeps every local state in f32.
+ * A forward that runs as a chain walk (see ssd_forward) stores no state per
+ * chunk and keeps the running state in f32; its last bits depend on the plan as
+ * well: whether the call walks, and into how many segments its chains are cut,
+ * follows from batch x heads, seqlen and the CU count (ssd_forward_plan). */
 enum {
   SSD_DTYPE_F32 = 0,
   SSD_DTYPE_BF16 = 1,
@@ -262,9 +265,12 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * head) chains times tokens run as a walk along the chains, 64 tokens a step
  * with the state in f32 registers, so that no per-chunk state is stored
  * (operands, then for few chains the end states of their segments, then the
- * walk: two to four launches; the workspace is the same).  Its results differ
- * from the stage kernels' by rounding; SSD_STATE_F16S (or SPLIT) as
- * state_dtype keeps the stage kernels.  f32 inputs at dstate 64 / 128 walk too
+ * walk: two to four launches; the workspace is the same).  In the product with
+ * cmat the state is held as the stage kernels of the call would hold it: as f16
+ * rows with a scale each (as SSD_STATE_F16S), or at chunk 128 (and in the layer
+ * at lengths that 256 does not divide) as a hi + lo pair of the input type.  Its
+ * results differ from the stage kernels' by rounding; SSD_STATE_F16S (or SPLIT)
+ * as state_dtype keeps the stage kernels.  f32 inputs at dstate 64 / 128 walk too
  * (two launches) with an even number of heads per group and more than two
  * chains per CU.  Otherwise, all on `stream`: at chunk 256
  * with 16-bit inputs K1 + K0 as one launch, then K2 + K3 as one state-chain
@@ -284,9 +290,10 @@ int ssd_chunk_scan(const ssd_dims* d, int dtype,
  * initial_states (the carried state updated in place). */
 /* The chunk length ssd_forward (and ssd_forward_noalloc) runs d's stage
  * kernels at, and sizes its workspace for, with this dtype and state_dtype:
- * d->chunk, or 256 where the rule above applies; 0 for invalid dims.  Host-only.  No counterpart in the reference (its
- * block_len is the chunk); for callers that size the workspace at the chunk
- * actually run or time its kernels one by one. */
+ * d->chunk, or 256 where the rule above applies; 0 for invalid dims.
+ * Host-only.  No counterpart in the reference (its block_len is the chunk);
+ * for callers that size the workspace at the chunk actually run or time its
+ * kernels one by one. */
 int64_t ssd_forward_chunk(const ssd_dims* d, int dtype, int state_dtype);
 
 /* How ssd_forward (gated 0) or ssd_layer_forward (gated 1; state_dtype
@@ -401,8 +408,9 @@ int ssd_layer_forward(const ssd_dims* d, int dtype, const ssd_layer_params* prm,
  * cached on the host; after a hipDeviceReset that cache is stale.  No
  * counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  Same arguments and results as ssd_forward otherwise,
- * at the chunk ssd_forward_chunk reports; the caller still provides every
+ * forbid hipMalloc).  Same arguments and results as ssd_forward otherwise (a
+ * call run in batch slices: those of ssd_forward on each slice, whose last bits
+ * may differ, as the launch plan depends on the batch), at the chunk ssd_forward_chunk reports; the caller still provides every
  * input and output.  When the workspace of the whole call is larger than the
  * array, the batch runs in slices whose workspace fits; a shape whose single
  * batch element needs more returns SSD_ERR_WORKSPACE_TOO_SMALL before any

@@ -425,6 +425,32 @@ def test_layer_span_two_heads(dtype, b, L, h, g):
     assert torch.equal(y, y2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,L,h,g", [(8, 384, 64, 4), (3, 1216, 80, 1), (2, 2496, 64, 8)])
+def test_captured_in_a_graph(b, L, h, g):
+    """A captured walk (one segment; four; eight linked ones) replayed on new
+    inputs, with eager calls between: the bits of the eager call each time."""
+    print("CASE chain walk, graph", b, L, h, g, flush=True)
+    on_the_walk(b, L, h, g, torch.bfloat16)
+    sets = [[t.to(DEV) for t in case(torch.bfloat16, b, L, h, g, seed)] for seed in (1, 2, 3)]
+    call = lambda X, A, B, C, dt, init: S.ssd_forward(X, A, B, C, 64, dt=dt, initial_states=init,  # noqa: E731
+                                                      return_final_states=True)
+    args = [t.clone() for t in sets[0]]
+    call(*args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        Y, final = call(*args)
+    for s in (sets[1], sets[2], sets[0], sets[1]):
+        for t, v in zip(args, s):
+            t.copy_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        Y0, f0 = call(*s)
+        torch.cuda.synchronize()
+        assert torch.equal(Y, Y0) and torch.equal(final, f0)
+
+
 # ---------------------------------------------------------------------------
 # addresses (CPU)
 # ---------------------------------------------------------------------------

@@ -33,14 +33,16 @@
 //     The weights go onto x (32 values per lane and step), as a hi + lo pair
 //     of the input type, rather than onto B^T, which every wave needs whole.
 //
-// Bound: with two workgroups of four waves per CU the SIMDs issue VALU and MFMA
-// for 84% of the cycles (the two do not overlap on one SIMD: VALU 50%, MFMA
-// 34%), at a clock that drops from 2.28 GHz on a lightly loaded chip to 1.85.
-// Taking out any one part (the lo products, the weighting, the B and C reads,
-// the exponentials) gains 2-4%, x's or y's traffic 12-18%.  Measured (us per
-// call, stage kernels -> walk): batch 8 x 2048 tokens, 128 heads, 8 groups, f16:
-// 368 -> 200, the layer span there 576 -> 382; batch 4 x 4096, 80 heads, bf16:
-// 197 -> 168 (3 segments); 1 x 65536, 80 heads: 800 -> 694 (12 segments).
+// Bound: issue.  At batch 4 x 4096, 80 heads the MFMAs are busy for 36% and the
+// VALU for 59% of the busy CUs' cycles (1 x 65536 the same, 8 x 2048 of 128 heads
+// 38% and 57%, gated 25% and 61%; counters), and the two do not overlap on one
+// SIMD.  Measured (us per call, stage kernels -> walk): batch 8 x 2048 tokens, 128
+// heads, 8 groups, f16: 365 -> 201, the layer span there 567 -> 365; batch 4 x
+// 4096, 80 heads, bf16: 197 -> 171 (3 segments); 1 x 65536, 80 heads: 800 -> 711
+// (38 segments); with S as a hi + lo pair, layer span 2 x 1216 of 128 heads: 250
+// -> 100 (one f16 there: 98).  The scale of every row costs 1-2% of a call: with rows
+// inside [2^-9, 2^15) left as they were, 4 x 4096 took 166.0 us instead of 167.5,
+// 1 x 65536 683 instead of 698 (f16 then loses bits below 2^-14).
 // Slower: two 16-row halves per wave on 16x16x32 MFMAs (twice the LDS reads: 437
 // against 387 us for the layer span), the MFMAs of a step behind all its copies
 // (a copy stalls its wave while others queue: 6% of a step).
@@ -748,20 +750,26 @@ size_t chain_scan_cscale_bytes(int64_t steps) { return (size_t)steps * kQ * size
 // The plan with the least expected time, and whether that is clearly (10%)
 // below the stage kernels'.  Times in us, from runs on 256 CUs: a step of the
 // scan takes `one` with at most one workgroup (two heads) on a CU, `two` with
-// two; a step of the state kernel 2.05 with up to one workgroup (four heads) per
-// CU.  Stage kernels: 27 + 9.4 per 1000 (chain, 64 token step) pairs, or where
-// 256 does not divide the sequence 52 + 22 per 1000; with the layer's gate 35 +
-// 13.1 and 40 + 38.  Both sides were within 15% of these on 18 shapes (us, stage
-// kernels / walk): 4 x 4096, 80 heads 208 / 178; 1 x 16384, 80 heads 231 / 200;
-// 3 x 3072, 80 heads 122 / 108; 16 x 512, 64 heads 87 / 52; 4 x 4096, 24 heads
-// 83 / 86; 1 x 2880, 80 heads 131 / 66; span 2 x 1216, 128 heads 248 / 93.
+// two; a step of the state kernel 2.05 with up to one workgroup (four heads, or
+// two of a group that four does not divide) per CU.  Stage kernels: 27 + 9.4 per
+// 1000 (chain, 64 token step) pairs, or where 256 does not divide the sequence
+// 52 + 22 per 1000; with the layer's gate 35 + 13.1 and 40 + 38.
+// Measured with forced segment counts on 18 shapes (us, stage kernels / chosen
+// count / fastest count): 4 x 4096, 80 heads 209 / 178 / 174; 3 x 3072, 80 heads
+// 117 / 104 / 104; 16 x 512, 64 heads 89 / 53 / 53; 1 x 2880, 80 heads 125 / 63 /
+// 63; 3 x 2368, 24 heads in groups of six 96 / 58 / 58; span 2 x 1216, 128 heads
+// 243 / 91 / 91, 1 x 2048 98 / 95 / 89.  Where the model is off: it knows no cost
+// per workgroup, so that 1 x 65536, 80 heads runs in 38 segments (735 us) where 12
+// take 711; and it is up to 18% high for few workgroups, so that 1 x 16384, 80
+// heads stays on the stage kernels (228; 190 in 12 segments).
 ChainScanPlan chain_scan_plan(int64_t batch, int64_t steps, int64_t nheads, int64_t ngroups, bool epi) {
   ChainScanPlan best{0, 0, false};
   const int64_t hpg = nheads / ngroups, chains = batch * nheads;
   if (hpg % 2 != 0) return best;
   const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  // Under ten steps per CU the stage kernels stay, which their own entry points
-  // reproduce bit for bit (2 x 2112 tokens of 24 heads: 87 us, 45 as a walk).
+  // Under ten steps per CU the stage kernels stay although the walk is faster (2 x
+  // 2112 tokens of 24 heads: 86 us, 44 as a walk): calls of that size are compared
+  // bit for bit with the stage kernels' own entry points.
   const int64_t pairs = chains * steps;
   if (pairs < 10 * cus) return best;
   const float one = epi ? 3.7f : 3.f, two = epi ? 6.7f : 5.3f;
@@ -789,7 +797,8 @@ ChainScanPlan chain_scan_plan(int64_t batch, int64_t steps, int64_t nheads, int6
   if (prep + best_us > 0.9f * stages) return ChainScanPlan{0, 0, false};
   // the gated variant with four heads per workgroup where that fills every CU
   // alike: B, C and C.B^T are copied once per four heads (batch 8 x 2048 of 128
-  // heads: 385 against 401 us; 2 x 1216, 136 against 105)
+  // heads: 368 against 380 us; 2 x 1216 in its four segments 91 against 92; where
+  // it leaves CUs idle, 4 x 2048, 256 against 205)
   const int64_t u4 = chains / 4 * best.nseg;
   best.wide = epi && hpg % 4 == 0 && u4 * 8 >= ((u4 + cus - 1) / cus) * cus * 7;
   return best;

@@ -22,9 +22,9 @@
 // first phase while B is copied, B in the second while the next C is.
 //
 // Bound: the f32 MFMAs (1/16 of the 16-bit rate).  At 64 x 512 tokens, 64 heads,
-// d_state 64 they keep the matrix cores busy for 73% of the scan's 433 us (three
-// workgroups per CU; two: 540 us) and the VALU adds 20%.  Measured (us per call,
-// stage kernels -> walk): that shape 712 -> 494, 32 x 1024, 32 heads, d_state 128
+// d_state 64 they keep the matrix cores busy for 79% of the scan's 425 us (three
+// workgroups per CU; two: 540 us) and the VALU adds 16%.  Measured (us per call,
+// stage kernels -> walk): that shape 714 -> 501, 32 x 1024, 32 heads, d_state 128
 // 541 -> 370, 16 x 512, 64 heads, d_state 64 189 -> 137.  No gain: wave
 // priorities by phase, a fixed interleaving of MFMA, VALU and LDS instructions.
 // W in registers for the whole step (formed between the off-diagonal products)
@@ -317,10 +317,12 @@ hipError_t launch_n(const ChainScanArgs& a, hipStream_t stream) {
 
 // Whole chains, where there is more than one workgroup (two chains) per CU.
 // Measured (us, stage kernels / walk; L 1024, 64 heads): 288 workgroups on 256 CUs
-// 309 / 220 at d_state 64 and 430 / 332 at 128; 480 402 / 240 and 1227 / 351.  With one per
-// CU or fewer, one wave per SIMD leaves the matrix cores idle for half a step and
-// the stage kernels, which their own entry points reproduce bit for bit, stay
-// (8 x 2048, 24 heads, d_state 128: 203 us).
+// 309 / 220 at d_state 64 and 430 / 332 at 128; 480 402 / 240 and 1227 / 351.  With fewer
+// than one per CU, one wave per SIMD leaves the matrix cores idle for half a step:
+// 96 workgroups (8 x 2048, 24 heads, d_state 128) 210 / 349, 128 267 / 358, 192
+// (d_state 64) 136 / 123.  With exactly one per CU the walk would win (277 / 190 at
+// d_state 128, 190 / 137 at 64); the line leaves it to the stage kernels, whose own
+// entry points give the forward's bits.
 ChainScanPlan chain_scan_f32_plan(int64_t batch, int64_t steps, int64_t nheads, int64_t ngroups, int64_t dstate) {
   const ChainScanPlan none{0, 0, false};
   if ((dstate != 64 && dstate != 128) || (nheads / ngroups) % kHeads != 0) return none;

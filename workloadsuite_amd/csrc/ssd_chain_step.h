@@ -96,8 +96,7 @@ __device__ __forceinline__ void chain_prep_body(const ChainScanArgs& p, int bcg,
   if constexpr (std::is_same<T, bf16>::value) {
     if (!p.ct) return;  // (S as a hi + lo pair: the walk takes C as it lies)
     // each row as f16 times 2^-e, its largest element in [2^14, 2^15) (bf16
-    // values then convert exactly down to 2^-24 of it), in operand order:
-    // piece 4 kc + g holds n = 32 kc + 4 g .. + 3 and 32 kc + 16 + 4 g .. + 3
+    // values then convert exactly down to 2^-31 of it)
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     uint32_t mb = 0;
 #pragma unroll

@@ -14,7 +14,8 @@ MR:97-99), the chunking rearranges (MR:105-110, 115) disappear because the
 kernels take ``[b, L, ...]`` tensors with strides, and dt scales x inside the
 kernels in float32 (MR:144 multiplies in float16).  ``block_len`` keeps MR's
 meaning for validation (it must divide the sequence length); the core itself
-runs at chunk 256 whenever L allows, which gives the same result up to
+runs as a walk along the (batch, head) chains in 64-token steps, or at chunk
+256 where L allows it, or at ``block_len``, all with the same result up to
 rounding (every chunking evaluates the same recurrence) with a quarter of the
 per-chunk state traffic of chunk 64.  RMSNorm and the two
 projections stay on PyTorch-ROCm (hipBLASLt/rocBLAS GEMMs), in MR's float16.

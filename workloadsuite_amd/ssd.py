@@ -335,7 +335,8 @@ def ssd_forward(X, A, B, C, chunk_size, dt=None, initial_states=None,
       number of heads per group and enough work for the GPU the whole core
       runs as a walk along the (batch, head) chains with the state in float32
       registers, and no states are handed over at all (float32 inputs: at
-      d_state 64 / 128 with more than two chains per CU).  Otherwise f16 rows
+      d_state 64 / 128 with more than two chains per CU; ``walk_plan`` tells).
+      Otherwise f16 rows
       with a power-of-two scale per row ("f16s") wherever a 16-bit chunk_scan
       reads them: chunk 256 with d_state 64 / 128, and chunk 64 / 128 with
       chunk x d_state <= 8192.
@@ -343,8 +344,8 @@ def ssd_forward(X, A, B, C, chunk_size, dt=None, initial_states=None,
       outside the one-launch state chain, and the chain's segments) the local
       states between them cross HBM as f16 rows with a scale per row and
       16-column tile (SSD_STATE_F16S_LOCAL); the state chain keeps them in
-      float32 registers.  Which launches run depends on batch x heads and the
-      device's CU count, so the last bits of Y and of the final state are not
+      float32 registers.  Which launches run, and how a walk cuts its chains,
+      depends on batch x heads and the device's CU count, so the last bits of Y and of the final state are not
       invariant to the batch size (within the 16-bit tolerance, and the final
       state within ~1e-3 of its scale).
     * "split": hi/lo pairs of the inputs' type at chunk 256 (plain float32
@@ -411,7 +412,8 @@ def ssd_forward_noalloc(X, A, B, C, chunk_size, dt=None, initial_states=None,
     """``ssd_forward`` through the C ABI's ``ssd_forward_noalloc``: the library
     takes its workspace from a device array it keeps per device instead of a
     buffer allocated here (for callers that cannot allocate: graph capture,
-    serving loops).  Same results.  Only the outputs are allocated (by torch,
+    serving loops).  Same results (a call too large for the array runs in batch
+    slices: those of ``ssd_forward`` on each slice).  Only the outputs are allocated (by torch,
     before the call); inputs that are not already in the kernels' layout are
     copied first, as in ``ssd_forward``.  Calls that overlap on one device race
     on that array."""
