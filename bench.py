@@ -638,9 +638,11 @@ def main():
 
     # each kernel alone, back to back on its own inputs
     for name, fn in kfn.items():
+        # (one row instead of five or six: more launches of it, for the start-up ramp below)
+        reps = args.kernel_reps * (4 if name == "chain_walk" else 1)
         fn()
-        kernels[name] = kernel_entry(name, time_launches(fn, args.kernel_reps))
-        pre_launches += 1 + args.kernel_reps
+        kernels[name] = kernel_entry(name, time_launches(fn, reps))
+        pre_launches += 1 + reps
 
     # ---- K forwards timed one by one: per-step median / mean / p90 / p99 ----
     # A fresh process's first ~60 forwards run slower (C3, per 20 steps after
@@ -727,7 +729,8 @@ def main():
         # warmup forwards
         "pre_timing": {"kernel_launches": pre_launches, "step_stats_forwards": pre_launches_forwards,
                        "warmup_forwards": args.warmup,
-                       "effective_warmup_forwards": pre_launches_forwards + args.warmup},
+                       # (a chain walk's or one-launch forward's timing launches are forwards too)
+                       "effective_warmup_forwards": pre_launches_forwards + args.warmup + (pre_launches if walk or small else 0)},
         "roofline": roof,
         "end_to_end": {"F_min_per_token": f_min / cfg.tokens, "B_min_per_token": b_min / cfg.tokens,
                        "roofline_tokens_per_s": roof_tps, "frac": round(tokens_per_s / roof_tps, 4)},
